@@ -181,11 +181,15 @@ int sp_sort_dropped_positions(uint64_t* count, int32_t reset);
  * counts[k] = number of entries; npl[k] = counts[k] for k < npl_limit, else 0
  * (npl nullable).  Serves the Native [2, kv, N] format (pos = input rows,
  * val = output rows: _scatter_pairs_native + native_pairs, pairs.py:223-278)
- * and the compacted weight-gradient signal (gemm.py:661-669). */
+ * and, without the tails, the compacted weight-gradient signal (gemm.py:661-669). */
 size_t sp_compact_workspace_size(int64_t kv, int64_t n);
 int sp_compact_table(const int32_t* table, int64_t kv, int64_t n, int32_t* pos_out,
                      int32_t* val_out, int32_t* counts, int32_t* npl, int32_t npl_limit,
                      void* ws, size_t ws_bytes, void* stream);
+
+/* The same without the -1 tails (counts required): the lists of sp_conv_wgrad. */
+int sp_compact_pairs(const int32_t* table, int64_t kv, int64_t n, int32_t* pos_out,
+                     int32_t* val_out, int32_t* counts, void* ws, size_t ws_bytes, void* stream);
 
 /* Native pair tensor [2, kv, n_pairs] -> gather tables.  pf [kv, n_out]
  * (-1 filled), pb [kv, n_in] (nullable).  inverse swaps the two rows of the
@@ -357,10 +361,11 @@ int sp_conv_dgrad(const void* g, int32_t dtype, int64_t n_out, int64_t K,
 int sp_split_bf16x3(const float* x, int64_t rows, int64_t cols, int32_t pattern, void* out,
                     void* stream);
 
-/* Weight gradient over compacted pairs (sp_compact_table of pair_fwd):
+/* Weight gradient over compacted pairs (sp_compact_pairs of pair_fwd):
  * dW[n, k, c] = sum_{p < counts[k]} X[in_rows[k, p], c] * G[out_rows[k, p], n].
- * X [n_in, C], G [n_out, K]; in_rows/out_rows [kv, row_stride].  Split-P fp32 partials reduced in a fixed
- * order (deterministic).  dW [K, kv, C] in dtype.  dtype SP_BF16X3: x [n_in, 2C]
+ * X [n_in, C], G [n_out, K]; in_rows/out_rows [kv, row_stride].  fp32 partials of
+ * shares of the pairs, summed in a fixed order (deterministic).  dW [K, kv, C] in dtype.
+ * dtype SP_BF16X3: x [n_in, 2C]
  * and g [n_out, 2K] are the bf16 [hi | lo] halves of fp32 tensors (sp_split_bf16x3
  * pattern 2), dW is fp32 (the four half products summed), and the workspace is
  * sp_wgrad_workspace_size(2K, kv, 2C, n_rows).

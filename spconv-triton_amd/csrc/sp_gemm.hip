@@ -30,8 +30,9 @@
 // compacted pairs of that offset.  The pair dimension is the MFMA reduction
 // dimension, so gathered rows are staged in LDS transposed ([channel][pair])
 // and read back as 16-byte MFMA operands.  The pair list of each offset is cut
-// into `splits` contiguous ranges whose fp32 partials are summed in a fixed
-// order by a second kernel (deterministic, no atomics).
+// into contiguous shares of about as many pairs for all offsets, whose fp32
+// partials are summed in a fixed order by a second kernel (deterministic, no
+// atomics).
 #include <mutex>
 #include <type_traits>
 
@@ -172,18 +173,43 @@ __device__ __forceinline__ typename Mfma<T>::frag load_frag_vec(const T* p) {
 // weight gradient
 // ---------------------------------------------------------------------------
 // dW[n, k, c] = sum over the pairs (i, o) of offset k of X[i, c] * G[o, n]:
-// per offset a GEMM whose reduction runs over that offset's compacted pair
-// list.  A workgroup owns (offset k, a contiguous share of its pairs, a
-// BW x BW block of (c, n)); each wave a BW/2 x BW/2 block of 32x32 MFMA tiles.
-// The MFMA operands need the pair index as the reduction index, i.e. X and G
-// transposed, so the rows gathered for a stage of pairs are written to LDS as
-// [channel][pair] (two pairs per write) and read back as 16-byte fragments.
-// Gathers are 16-byte vector loads; the next stage's rows and the pair indices
-// two stages ahead are in flight while the stage's MFMAs run.  Every (c, n)
-// block gathers the rows of all its pairs again, so wide layers take
-// BW = 128: half the gathered bytes of BW = 64 at C, K >= 128.
-// fp32 partials per share are summed in a fixed order by wgrad_reduce
-// (deterministic, no atomics).
+// per offset a GEMM whose reduction runs over that offset's pairs, in
+// ascending output row.  A workgroup owns (offset k, a contiguous share of its
+// pairs, a BW x BW block of (c, n)); each wave a BW/2 x BW/2 block of 32x32
+// MFMA tiles.  The MFMA operands need the pair index as the reduction index,
+// i.e. X and G transposed, so the rows gathered for a stage of pairs are
+// written to LDS as [channel][pair] (two pairs per write) and read back as
+// 16-byte fragments.  Gathers are 16-byte vector loads; the next stage's rows
+// are in flight while the stage's MFMAs run.  Every (c, n) block gathers the
+// rows of all its pairs again, so wide layers take BW = 128: half the gathered
+// bytes of BW = 64 at C, K >= 128.
+//
+// Shares.  Offsets differ widely in pairs (the centre of a sparse submanifold
+// table holds more than all others together), so an offset gets a share per
+// `per` of its pairs, `per` a whole number of stages and the same for all
+// offsets: all workgroups run about as long.  The fp32 partial of each share
+// is summed in ascending share by wgrad_reduce (deterministic, no atomics).
+//
+// Pairs per share: the total over `target` shares, in whole stages.
+__device__ __forceinline__ int64_t wg_per(int64_t total, int target, int stage) {
+  const int64_t stages = (total + int64_t(target) * stage - 1) / (int64_t(target) * stage);
+  return (stages > 0 ? stages : 1) * stage;
+}
+
+// Sum over the workgroup's NT threads, in a fixed order; red holds NT / 64.
+template <int NT>
+__device__ __forceinline__ int64_t wg_block_sum(int64_t v, int64_t* red) {
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  int64_t t = 0;
+#pragma unroll
+  for (int w = 0; w < NT / 64; ++w) t += red[w];
+  __syncthreads();
+  return t;
+}
+
 template <typename T, int BW>
 struct WgShape {
   static constexpr int kStage = BW == 64 || sizeof(T) == 2 ? 128 : 64;  // pairs per LDS stage
@@ -203,8 +229,8 @@ template <typename T, int VEC, int BW>
 __global__ __launch_bounds__(256) void wgrad_partial(
     const T* __restrict__ X, int64_t n_in, const T* __restrict__ G, int64_t n_out, int C, int K,
     int kv, const int32_t* __restrict__ in_rows, const int32_t* __restrict__ out_rows,
-    const int32_t* __restrict__ counts, int64_t stride, int splits, float* __restrict__ part,
-    uint32_t x_bytes, uint32_t g_bytes, int cblocks, int nblocks) {
+    const int32_t* __restrict__ counts, int64_t stride, int target, int slots,
+    float* __restrict__ part, uint32_t x_bytes, uint32_t g_bytes, int cblocks, int nblocks) {
   using MF = Mfma<T>;
   using frag = typename MF::frag;
   using S = WgShape<T, BW>;
@@ -228,18 +254,42 @@ __global__ __launch_bounds__(256) void wgrad_partial(
     return COAL ? ((((p >> 3) ^ (((c >> 4) & 1) << 2)) << 3) | (p & 7)) : p;
   };
 
-  // (offset, split) pair ks and (c, n) block of this workgroup: the
-  // cblocks * nblocks blocks of one pair gather the same pairs' rows (each
-  // input row for every n block, each gradient row for every c block), so
-  // they run back to back on one XCD (workgroup b runs on XCD b % 8) and the
-  // second reader of a row finds it in that XCD's L2
+  __shared__ int64_t s_red[4];
+  __shared__ uint32_t s_scan[5];
+  __shared__ int s_found[2];
+
+  // share `slot` and (c, n) block of this workgroup: the cblocks * nblocks
+  // blocks of one share gather the same pairs' rows (each input row for every
+  // n block, each gradient row for every c block), so they run back to back on
+  // one XCD (workgroup b runs on XCD b % 8) and the second reader of a row
+  // finds it in that XCD's L2
   const int bpk = cblocks * nblocks;
   const int64_t t = blockIdx.x / 8;
-  const int64_t ks = (t / bpk) * 8 + blockIdx.x % 8;
-  if (ks >= int64_t(kv) * splits) return;  // padding of the last group of 8 pairs
+  const int slot = int((t / bpk) * 8 + blockIdx.x % 8);
+  if (slot >= slots) return;  // padding of the last group of 8 shares
   const int blk = int(t % bpk);
-  const int k = int(ks / splits);
-  const int split = int(ks % splits);
+  int64_t total = 0;
+  for (int kk = threadIdx.x; kk < kv; kk += 256) total += counts[kk];
+  total = wg_block_sum<256>(total, s_red);
+  const int64_t per = wg_per(total, target, STAGE);
+  if (threadIdx.x == 0) s_found[0] = -1;
+  uint32_t before = 0;
+  for (int kb = 0; kb < kv; kb += 256) {  // the offset whose shares hold `slot`
+    const int kk = kb + int(threadIdx.x);
+    const uint32_t ns = kk < kv ? uint32_t((counts[kk] + per - 1) / per) : 0u;
+    uint32_t all;
+    const uint32_t lo = before + block_exclusive_scan<256>(ns, s_scan, &all);
+    if (uint32_t(slot) >= lo && uint32_t(slot) < lo + ns) {
+      s_found[0] = kk;
+      s_found[1] = slot - int(lo);
+    }
+    before += all;
+    if (uint32_t(slot) < before) break;
+  }
+  __syncthreads();
+  const int k = s_found[0];
+  if (k < 0) return;  // fewer shares than slots
+  const int split = s_found[1];
   const int c0 = (blk / nblocks) * BW, n0 = (blk % nblocks) * BW;
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
@@ -253,9 +303,8 @@ __global__ __launch_bounds__(256) void wgrad_partial(
   auto ch_of = [&](int j) -> int { return COAL ? j * 4 * V + q * V : q * S::kCh + j * V; };
 
   const int64_t cnt = counts[k];
-  const int64_t chunk = (cnt + splits - 1) / splits;
-  const int64_t p_lo = split * chunk;
-  const int64_t p_hi = p_lo + chunk < cnt ? p_lo + chunk : cnt;
+  const int64_t p_lo = split * per;
+  const int64_t p_hi = p_lo + per < cnt ? p_lo + per : cnt;
 
   const __amdgpu_buffer_rsrc_t rx = make_rsrc(X, x_bytes);
   const __amdgpu_buffer_rsrc_t rg = make_rsrc(G, g_bytes);
@@ -353,47 +402,103 @@ __global__ __launch_bounds__(256) void wgrad_partial(
     }
   }
   // D[c][n]: lane holds column n = l32 of rows c = 8*(i/4) + 4*h + (i%4)
+  float* ps = part + int64_t(slot) * K * C;
 #pragma unroll
   for (int mc = 0; mc < MT; ++mc)
 #pragma unroll
     for (int mn = 0; mn < MT; ++mn) {
       const int n = n0 + ntile + 32 * mn + l32;
 #pragma unroll
-      for (int i = 0; i < 16; ++i) {
-        const int c = c0 + ctile + 32 * mc + (i >> 2) * 8 + h * 4 + (i & 3);
-        if (c < C && n < K) part[((int64_t(split) * K + n) * kv + k) * C + c] = acc[mc][mn][i];
+      for (int i = 0; i < 16; i += 4) {
+        const int c = c0 + ctile + 32 * mc + (i >> 2) * 8 + h * 4;
+        if (n >= K) continue;
+        float* d = ps + int64_t(n) * C + c;
+        if (c + 3 < C && C % 4 == 0) {
+          *reinterpret_cast<float4*>(d) = make_float4(acc[mc][mn][i], acc[mc][mn][i + 1],
+                                                      acc[mc][mn][i + 2], acc[mc][mn][i + 3]);
+        } else {
+#pragma unroll
+          for (int e = 0; e < 4; ++e)
+            if (c + e < C) d[e] = acc[mc][mn][i + e];
+        }
       }
     }
 }
 
-template <typename T>
-__global__ void wgrad_reduce(const float* __restrict__ part, int splits, int64_t total,
-                             T* __restrict__ dw) {
-  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= total) return;
-  float s = 0.f;
-  for (int p = 0; p < splits; ++p) s += part[int64_t(p) * total + i];
-  dw[i] = from_f32<T>(s);
-}
+// dW of one offset from its shares' partials [slot][n][c], W = 4 (whole 16-byte
+// pieces) or 1 values a lane.  The workgroup's NW waves each sum a contiguous
+// part of the offset's shares, eight in flight, and the sums meet in LDS in
+// ascending share.  SPLIT: the partials hold the products of X's and G's
+// [hi | lo] halves ([2K][2C]), whose four values of an entry are added, in a
+// fixed order, into the fp32 dW.
+template <typename T, int W, bool SPLIT, int NW>
+__global__ __launch_bounds__(64 * NW) void wgrad_reduce(
+    const float* __restrict__ part, const int32_t* __restrict__ counts, int kv, int target,
+    int stage, int K, int C, T* __restrict__ dw) {
+  __shared__ float s_part[NW][64 * W];
+  __shared__ int64_t s_red[NW];
+  const int k = int(blockIdx.y);
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  int64_t total = 0;
+  for (int kk = threadIdx.x; kk < kv; kk += 64 * NW) total += counts[kk];
+  const int64_t per = wg_per(wg_block_sum<64 * NW>(total, s_red), target, stage);
+  int64_t lo = 0;  // the offset's first share
+  for (int kk = threadIdx.x; kk < k; kk += 64 * NW)
+    lo += (counts[kk] + per - 1) / per;
+  lo = wg_block_sum<64 * NW>(lo, s_red);
+  const int ns = int((counts[k] + per - 1) / per);
 
-// The weight gradient of split-bf16 operands (SP_BF16X3): the partials hold
-// [2K][kv][2C] = the four products of X's and G's [hi | lo] halves, which are
-// summed in a fixed order into the fp32 dW [K][kv][C].
-__global__ void wgrad_reduce_split(const float* __restrict__ part, int splits, int64_t K,
-                                   int64_t kv, int64_t C, float* __restrict__ dw) {
-  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int64_t total = K * kv * C;
-  if (i >= total) return;
-  const int64_t c = i % C, nk = i / C, k = nk % kv, n = nk / kv;
-  const int64_t part_total = 4 * total;
-  float s = 0.f;
-  for (int p = 0; p < splits; ++p)
+  const int E = K * C;
+  const int e0 = (int(blockIdx.x) * 64 + lane) * W;
+  const bool ok = e0 < E;
+  const int each = (ns + NW - 1) / NW;
+  const int w_lo = wave * each < ns ? wave * each : ns;
+  const int w_hi = w_lo + each < ns ? w_lo + each : ns;
+  using vec = __attribute__((ext_vector_type(W))) float;
+  const int64_t pitch = SPLIT ? 4 * int64_t(E) : int64_t(E);  // floats of a share
+  constexpr int kParts = SPLIT ? 4 : 1;
+  int64_t at[kParts];
+  if constexpr (SPLIT) {
+    const int n = e0 / C, c = e0 % C;  // (W divides C)
 #pragma unroll
     for (int a = 0; a < 2; ++a)
 #pragma unroll
-      for (int b = 0; b < 2; ++b)
-        s += part[int64_t(p) * part_total + ((a * K + n) * kv + k) * 2 * C + b * C + c];
-  dw[i] = s;
+      for (int b = 0; b < 2; ++b) at[2 * a + b] = (int64_t(a) * K + n) * 2 * C + int64_t(b) * C + c;
+  } else {
+    at[0] = e0;
+  }
+  vec sum;
+#pragma unroll
+  for (int i = 0; i < W; ++i) sum[i] = 0.f;
+  if (ok) {
+    const float* p = part + (lo + w_lo) * pitch;
+    constexpr int kBatch = 8 / kParts;
+    int s = w_lo;
+    for (; s + kBatch <= w_hi; s += kBatch, p += kBatch * pitch) {
+      vec v[kBatch][kParts];
+#pragma unroll
+      for (int b = 0; b < kBatch; ++b)
+#pragma unroll
+        for (int q = 0; q < kParts; ++q)
+          v[b][q] = *reinterpret_cast<const vec*>(p + b * pitch + at[q]);
+#pragma unroll
+      for (int b = 0; b < kBatch; ++b)
+#pragma unroll
+        for (int q = 0; q < kParts; ++q) sum += v[b][q];
+    }
+    for (; s < w_hi; ++s, p += pitch)
+#pragma unroll
+      for (int q = 0; q < kParts; ++q) sum += *reinterpret_cast<const vec*>(p + at[q]);
+  }
+  *reinterpret_cast<vec*>(&s_part[wave][lane * W]) = sum;
+  __syncthreads();
+  if (wave != 0 || !ok) return;
+  for (int w = 1; w < NW; ++w) sum += *reinterpret_cast<const vec*>(&s_part[w][lane * W]);
+#pragma unroll
+  for (int i = 0; i < W; ++i) {
+    const int e = e0 + i, n = e / C, c = e % C;
+    dw[(int64_t(n) * kv + k) * C + c] = from_f32<T>(sum[i]);
+  }
 }
 
 // out [rows][parts * cols] bf16 from x [rows][cols] fp32: pattern 0 = [hi |
@@ -792,22 +897,30 @@ static int gemm_common(const void* A, int dtype, int64_t n_src, const void* w, i
 // (c, n) block width of the weight-gradient workgroups
 static int wgrad_block(int64_t C, int64_t K) { return C >= 128 && K >= 128 ? 128 : 64; }
 
-// Splits per (offset, block): 64 workgroups per offset (at least 512 in all), so that the
-// per-split fp32 partials (splits x kv x C x K x 4 bytes, written and read back) stay in
-// proportion to the gathered bytes.  Measured over the 12 calls of the ResUNet training step
-// (forced split counts 4..64 per call): the best count per call is close to 64 / blocks in
-// every call (the 256 -> 256 call at 16, the 64 -> 32 calls at 64), 1.14 -> 0.94 ms in all
-// against a target of 1 024 workgroups per call.
-static int wgrad_splits(int64_t kv, int64_t C, int64_t K, int64_t n_rows) {
+// Shares a call aims at, and the slots its partials need: an offset's last
+// share may be a short one, so there are at most kv more shares than aimed at.
+// fp32 results take 64 shares per offset (at least 512 workgroups in all), so
+// that no chain of fp32 sums is long; for 16-bit ones, whose rounding hides
+// that, the fewest that fill the chip: every share writes and reads a fp32
+// partial of its block.  Measured (us a call, 256 / 512 / 768 / 1024 / 1536 /
+// 2048 workgroups): urban 240k rows, 410k pairs, 64 -> 64 33.2 / 30.5 / 33.8 /
+// 35.4 / 37.1 / 42.4; k2 s2 64 -> 128 33.2 / 27.8 / 28.6 / 29.9 / 32.2 / 36.6;
+// 75k rows, 349k pairs, 256 -> 128 (128-wide blocks) 108 / 107 / 100 / 99 /
+// 108 / 117, 256 -> 256 189 / 183 / 165 / 166 / 166 / 176.
+static int wgrad_target(int64_t kv, int64_t C, int64_t K, int64_t n_rows, bool f32) {
   const int bw = wgrad_block(C, K);
-  const int64_t tiles = kv * cdiv(C, bw) * cdiv(K, bw);
-  const int64_t target = 64 * kv > 512 ? 64 * kv : 512;
-  int64_t splits = cdiv(target, tiles);
-  const int64_t by_len = cdiv(n_rows, 1024);    // keep >= ~1k rows of work per split
-  if (splits > by_len) splits = by_len;
-  if (splits > 64) splits = 64;
-  if (splits < 1) splits = 1;
-  return int(splits);
+  int64_t wgs = bw == 128 ? 1024 : 512;
+  if (f32 && wgs < 64 * kv) wgs = 64 * kv;
+  int64_t t = cdiv(wgs, cdiv(C, bw) * cdiv(K, bw));
+  const int64_t by_len = cdiv(n_rows * kv, 128);  // a stage of pairs each, if every entry were one
+  if (t > by_len) t = by_len;
+  return int(t < 1 ? 1 : t);
+}
+// Blocks up to this many values an offset are reduced by 16 waves a workgroup
+// (few workgroups, and a dense offset has most of the shares), larger ones by 4.
+constexpr int64_t kWgWideReduce = 8192;
+static int64_t wgrad_slots(int64_t kv, int64_t C, int64_t K, int64_t n_rows, bool f32) {
+  return wgrad_target(kv, C, K, n_rows, f32) + kv;
 }
 
 // ---- the forward without a caller workspace (sp_conv_fwd_noalloc) ---------
@@ -938,8 +1051,8 @@ int sp_conv_dgrad(const void* g, int32_t dtype, int64_t n_out, int64_t K, const 
 }
 
 size_t sp_wgrad_workspace_size(int64_t K, int64_t kv, int64_t C, int64_t n_rows) {
-  const int splits = wgrad_splits(kv, C, K, n_rows);
-  return align_up(size_t(splits) * size_t(K * kv * C) * sizeof(float), 256);
+  // (the larger of the two shares' counts: the type is not known here)
+  return align_up(size_t(wgrad_slots(kv, C, K, n_rows, true)) * size_t(K * C) * sizeof(float), 256);
 }
 
 int sp_conv_wgrad(const void* x, int64_t n_in, const void* g, int64_t n_out, int32_t dtype,
@@ -955,14 +1068,16 @@ int sp_conv_wgrad(const void* x, int64_t n_in, const void* g, int64_t n_out, int
   const bool split = dtype == SP_BF16X3;
   const int64_t Cg = split ? 2 * C : C, Kg = split ? 2 * K : K;
   SP_CHECK_ARG(Kg < 65536 && Cg < 65536 && kv < 65536, "wgrad: channel/kernel size too large");
+  SP_CHECK_ARG(Kg * Cg < (int64_t(1) << 30) && row_stride < (int64_t(1) << 31),
+               "wgrad: weight or table too large");
   const int elem = split ? SP_BF16 : dtype;
-  const int splits = wgrad_splits(kv, Cg, Kg, row_stride);
+  const bool f32 = split || elem == SP_F32;
+  const int64_t slots = wgrad_slots(kv, Cg, Kg, row_stride, f32);
+  const int target = wgrad_target(kv, Cg, Kg, row_stride, f32);
   const size_t need = sp_wgrad_workspace_size(Kg, kv, Cg, row_stride);
   if (!ws || ws_bytes < need)
     return set_error(SP_ERR_WORKSPACE, "wgrad: workspace %zu < %zu", ws_bytes, need);
   float* part = static_cast<float*>(ws);
-  const int64_t gx = kv * splits;
-  SP_CHECK_ARG(gx <= kMaxGridX, "wgrad: grid too large");
   const int64_t es = elem == SP_F32 ? 4 : 2;
   const int64_t xb = n_in * Cg * es, gb = n_out * Kg * es;
   if (xb >= int64_t(kOob) || gb >= int64_t(kOob))
@@ -973,11 +1088,11 @@ int sp_conv_wgrad(const void* x, int64_t n_in, const void* g, int64_t n_out, int
                   (Kg % v == 0 && reinterpret_cast<uintptr_t>(g) % 16 == 0 ? 2 : 0);
   const int bw = wgrad_block(Cg, Kg);
   const int cblocks = int(cdiv(Cg, bw)), nblocks = int(cdiv(Kg, bw));
-  const int64_t nwg = 8 * cdiv(gx, 8) * cblocks * nblocks;
+  const int64_t nwg = 8 * cdiv(slots, 8) * cblocks * nblocks;
   SP_CHECK_ARG(nwg <= kMaxGridX, "wgrad: grid too large");
   const dim3 grid{unsigned(nwg), 1u, 1u};
-  const int64_t tot = K * kv * C;
-  const unsigned rb = unsigned(cdiv(tot, 256));
+  const int rw = C % 4 == 0 ? 4 : 1;
+  const dim3 rgrid{unsigned(cdiv(K * C, 64 * rw)), unsigned(kv)};
   auto run = [&](auto tag) {
     using T = decltype(tag);
     using Kern = decltype(&wgrad_partial<T, 3, 64>);
@@ -988,11 +1103,27 @@ int sp_conv_wgrad(const void* x, int64_t n_in, const void* g, int64_t n_out, int
     const Kern kern = bw == 128 ? k128[vec] : k64[vec];
     kern<<<grid, 256, 0, s>>>(static_cast<const T*>(x), n_in, static_cast<const T*>(g), n_out,
                               int(Cg), int(Kg), int(kv), in_rows, out_rows, counts, row_stride,
-                              splits, part, uint32_t(xb), uint32_t(gb), cblocks, nblocks);
+                              target, int(slots), part, uint32_t(xb), uint32_t(gb), cblocks,
+                              nblocks);
+    const int stage = bw == 128 ? WgShape<T, 128>::kStage : WgShape<T, 64>::kStage;
+    auto reduce = [&](auto out, auto is_split, auto waves) {
+      using O = decltype(out);
+      constexpr bool SPL = decltype(is_split)::value;
+      constexpr int NW = decltype(waves)::value;
+      auto red = rw == 4 ? wgrad_reduce<O, 4, SPL, NW> : wgrad_reduce<O, 1, SPL, NW>;
+      red<<<rgrid, 64 * NW, 0, s>>>(part, counts, int(kv), target, stage, int(K), int(C),
+                                    static_cast<O*>(dw));
+    };
+    auto with_waves = [&](auto out, auto is_split) {
+      if (K * C <= kWgWideReduce)
+        reduce(out, is_split, std::integral_constant<int, 16>{});
+      else
+        reduce(out, is_split, std::integral_constant<int, 4>{});
+    };
     if (split)
-      wgrad_reduce_split<<<rb, 256, 0, s>>>(part, splits, K, kv, C, static_cast<float*>(dw));
+      with_waves(float{}, std::true_type{});
     else
-      wgrad_reduce<T><<<rb, 256, 0, s>>>(part, splits, tot, static_cast<T*>(dw));
+      with_waves(T{}, std::false_type{});
   };
   switch (elem) {
     case SP_F16: run(_Float16{}); break;

@@ -612,9 +612,9 @@ def compacted_signal(pair_fwd: torch.Tensor):
     counts = torch.empty((kv,), dtype=torch.int32, device=device)
     L = _lib.lib()
     ws = _lib.workspace(L.sp_compact_workspace_size(kv, n), device)
-    _lib.check(L.sp_compact_table(_lib.ptr(pf), kv, n, _lib.ptr(out_rows), _lib.ptr(in_rows),
-                                  _lib.ptr(counts), None, kv, _lib.ptr(ws), ws.numel(),
-                                  _lib.stream_of(device)), "sp_compact_table")
+    _lib.check(L.sp_compact_pairs(_lib.ptr(pf), kv, n, _lib.ptr(out_rows), _lib.ptr(in_rows),
+                                  _lib.ptr(counts), _lib.ptr(ws), ws.numel(),
+                                  _lib.stream_of(device)), "sp_compact_pairs")
     sig = (in_rows, out_rows, counts)
     pair_fwd._spconv_triton_dw_sig = sig
     return sig
@@ -622,7 +622,7 @@ def compacted_signal(pair_fwd: torch.Tensor):
 
 def conv_backward_weight(features: torch.Tensor, grad_out: torch.Tensor, pair_fwd: torch.Tensor,
                          weight_shape_krsc, fp32_accum: bool | None = None) -> torch.Tensor:
-    """dW [K, kv, C] = per-offset X^T G over compacted pairs (deterministic split-P)."""
+    """dW [K, kv, C] = per-offset X^T G over compacted pairs (deterministic shares)."""
     _lib.require_gpu(features, grad_out, pair_fwd)
     K, C = int(weight_shape_krsc[0]), int(weight_shape_krsc[-1])
     kv = int(pair_fwd.shape[0])

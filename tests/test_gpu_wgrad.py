@@ -1,0 +1,86 @@
+"""The weight gradient's pair compaction and shares at the sizes where they can
+go wrong: chunks and runs of the compaction cut short, offsets without pairs,
+one offset with nearly all of them, more offsets than a workgroup looks at in
+one turn, rows of no whole vector, and blocks on both sides of the reduction's
+two instances."""
+
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda"
+
+
+def _table(kv, n, n_in, density, seed):
+    """[kv, n] gather table; density of offset k: density[k % len(density)]."""
+    rng = np.random.default_rng(seed)
+    t = rng.integers(0, n_in, size=(kv, n), dtype=np.int32)
+    keep = rng.random((kv, n)) < np.asarray(density)[np.arange(kv) % len(density)][:, None]
+    return np.where(keep, t, -1).astype(np.int32)
+
+
+@pytest.mark.parametrize("kv,n,density", [
+    (1, 1, [1.0]), (3, 63, [0.0, 1.0, 0.3]), (27, 1024, [0.1]), (27, 1025, [0.02, 1.0]),
+    (8, 64 * 1024, [0.5]), (5, 65 * 1024 + 3, [0.001, 0.9]), (300, 700, [0.05, 0.0, 0.4])])
+def test_compaction_matches_numpy(kv, n, density):
+    from spconv_triton.pytorch._impl import _lib
+    from spconv_triton.pytorch._impl.gemm import compacted_signal
+
+    t = _table(kv, n, 1000, density, kv + n)
+    tab = torch.from_numpy(t).to(DEV)
+    in_rows, out_rows, counts = compacted_signal(tab)
+    # the same lists with -1 tails and limited counts (the Native format)
+    L = _lib.lib()
+    pos, val = torch.empty_like(tab), torch.empty_like(tab)
+    npl = torch.empty(kv, dtype=torch.int32, device=DEV)
+    ws = _lib.workspace(L.sp_compact_workspace_size(kv, n), tab.device)
+    _lib.check(L.sp_compact_table(_lib.ptr(tab), kv, n, _lib.ptr(pos), _lib.ptr(val), None,
+                                  _lib.ptr(npl), kv // 2, _lib.ptr(ws), ws.numel(),
+                                  _lib.stream_of(tab.device)), "sp_compact_table")
+    pos, val, npl = pos.cpu().numpy(), val.cpu().numpy(), npl.cpu().numpy()
+    in_rows, out_rows, counts = (v.cpu().numpy() for v in (in_rows, out_rows, counts))
+    for k in range(kv):
+        cols = np.nonzero(t[k] >= 0)[0]
+        m = cols.size
+        assert counts[k] == m and npl[k] == (m if k < kv // 2 else 0)
+        for got_pos, got_val in ((pos[k], val[k]), (out_rows[k], in_rows[k])):
+            np.testing.assert_array_equal(got_pos[:m], cols)
+            np.testing.assert_array_equal(got_val[:m], t[k, cols])
+        assert (pos[k, m:] == -1).all() and (val[k, m:] == -1).all()
+
+
+@pytest.mark.parametrize("kv,n,C,K,density,dtype", [
+    (27, 3000, 64, 64, [0.05], torch.float16),
+    (27, 40000, 64, 64, [0.001] * 13 + [1.0] + [0.001] * 13, torch.float16),  # a dense centre
+    (27, 40000, 160, 128, [0.001] * 13 + [1.0] + [0.001] * 13, torch.bfloat16),
+    (300, 500, 32, 16, [0.0, 0.2], torch.float32),  # more offsets than threads
+    (8, 129, 256, 256, [1.0], torch.float16),  # one stage and one pair
+    (27, 2000, 3, 20, [0.1], torch.float16),  # rows of no whole vector
+    (1, 1, 16, 16, [1.0], torch.float32),
+    (9, 5000, 72, 120, [0.3], torch.float32),
+    (2, 700, 5, 7, [0.0, 0.5], torch.float32),  # an offset without pairs, scalar reduction
+])
+def test_shares_match_fp64(kv, n, C, K, density, dtype):
+    """|error| <= (2 u_out + sum_depth 2^-24) * sum |x||g|: the result's own rounding and
+    fp32 sums no deeper than an offset's pairs."""
+    from spconv_triton.pytorch._impl.gemm import conv_backward_weight
+
+    n_in = n + 17
+    t = _table(kv, n, n_in, density, kv * 7 + n)
+    g = torch.Generator(device=DEV)
+    g.manual_seed(n)
+    x = torch.randn(n_in, C, generator=g, device=DEV).to(dtype)
+    go = torch.randn(n, K, generator=g, device=DEV).to(dtype)
+    tab = torch.from_numpy(t).to(DEV)
+    dw = conv_backward_weight(x, go, tab, (K, kv, C))
+    again = conv_backward_weight(x, go, tab, (K, kv, C))
+    assert torch.equal(dw, again)
+    unit = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8, torch.float32: 2.0 ** -24}[dtype]
+    for k in range(kv):
+        o = torch.nonzero(tab[k] >= 0).view(-1)
+        xi, gi = x[tab[k][o].long()].double(), go[o].double()
+        ref, mag = gi.T @ xi, gi.abs().T @ xi.abs()
+        bound = (2 * unit + min(o.numel(), 4096) * 2.0 ** -24) * mag + 1e-30
+        assert ((dw[:, k].double() - ref).abs() <= bound).all(), f"offset {k}"
