@@ -17,14 +17,6 @@ int set_error(int code, const char* fmt, ...) {
   return code;
 }
 
-// POPC: the values scanned are the population counts of the input words (the
-// ranks of set bits in a bitmap) rather than the words themselves.
-template <bool POPC>
-__device__ __forceinline__ uint32_t scan_value(uint32_t w) {
-  return POPC ? uint32_t(__popc(w)) : w;
-}
-
-template <bool POPC>
 __global__ __launch_bounds__(kScanThreads) void scan_chunk_sums(const uint32_t* __restrict__ in,
                                                                 int64_t len,
                                                                 uint32_t* __restrict__ sums) {
@@ -34,7 +26,7 @@ __global__ __launch_bounds__(kScanThreads) void scan_chunk_sums(const uint32_t* 
 #pragma unroll
   for (int i = 0; i < kScanItems; ++i) {
     int64_t idx = base + int64_t(i) * kScanThreads + threadIdx.x;
-    if (idx < len) s += scan_value<POPC>(in[idx]);
+    if (idx < len) s += in[idx];
   }
   uint32_t tot;
   block_exclusive_scan<kScanThreads>(s, lds, &tot);
@@ -63,7 +55,7 @@ __global__ __launch_bounds__(1024) void scan_sums_single(uint32_t* __restrict__ 
 // Each thread owns kScanItems consecutive counts of the chunk; with VEC4
 // (16-byte aligned arrays) a thread's whole counts move as 16-byte loads and
 // stores (one count per load had each instruction touch 64 lines).
-template <bool VEC4, bool POPC>
+template <bool VEC4>
 __global__ __launch_bounds__(kScanThreads) void scan_chunk_apply(const uint32_t* __restrict__ in,
                                                                  uint32_t* __restrict__ out,
                                                                  int64_t len,
@@ -91,10 +83,7 @@ __global__ __launch_bounds__(kScanThreads) void scan_chunk_apply(const uint32_t*
     }
   }
 #pragma unroll
-  for (int i = 0; i < kScanItems; ++i) {
-    v[i] = scan_value<POPC>(v[i]);
-    s += v[i];
-  }
+  for (int i = 0; i < kScanItems; ++i) s += v[i];
   uint32_t tot;
   uint32_t run = block_exclusive_scan<kScanThreads>(s, lds, &tot) + sums[blockIdx.x];
   uint32_t o[kScanItems];
@@ -120,34 +109,23 @@ size_t scan_workspace_bytes(int64_t len) {
   return align_up(size_t(chunks) * sizeof(uint32_t), 256);
 }
 
-template <bool POPC>
-static int exclusive_scan(const uint32_t* in, uint32_t* out, int64_t len, uint32_t* total,
-                          void* ws, hipStream_t stream) {
+int exclusive_scan_u32(const uint32_t* in, uint32_t* out, int64_t len, uint32_t* total,
+                       void* ws, hipStream_t stream) {
   if (len <= 0) return SP_OK;
   const int64_t chunks = cdiv(len, kScanChunk);
   uint32_t* sums = static_cast<uint32_t*>(ws);
-  scan_chunk_sums<POPC><<<dim3(unsigned(chunks)), dim3(kScanThreads), 0, stream>>>(in, len, sums);
+  scan_chunk_sums<<<dim3(unsigned(chunks)), dim3(kScanThreads), 0, stream>>>(in, len, sums);
   SP_LAUNCHED();
   scan_sums_single<<<dim3(1), dim3(1024), 0, stream>>>(sums, chunks, total);
   SP_LAUNCHED();
   if (((reinterpret_cast<uintptr_t>(in) | reinterpret_cast<uintptr_t>(out)) & 15) == 0)
-    scan_chunk_apply<true, POPC>
+    scan_chunk_apply<true>
         <<<dim3(unsigned(chunks)), dim3(kScanThreads), 0, stream>>>(in, out, len, sums);
   else
-    scan_chunk_apply<false, POPC>
+    scan_chunk_apply<false>
         <<<dim3(unsigned(chunks)), dim3(kScanThreads), 0, stream>>>(in, out, len, sums);
   SP_LAUNCHED();
   return SP_OK;
-}
-
-int exclusive_scan_u32(const uint32_t* in, uint32_t* out, int64_t len, uint32_t* total,
-                       void* ws, hipStream_t stream) {
-  return exclusive_scan<false>(in, out, len, total, ws, stream);
-}
-
-int exclusive_scan_popc(const uint32_t* words, uint32_t* out, int64_t len, uint32_t* total,
-                        void* ws, hipStream_t stream) {
-  return exclusive_scan<true>(words, out, len, total, ws, stream);
 }
 
 }  // namespace sp

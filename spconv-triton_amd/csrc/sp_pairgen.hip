@@ -23,6 +23,9 @@
 //    is written back into its hash slot as its output row.
 #include <type_traits>
 
+#include <mutex>
+#include <vector>
+
 #include "sp_common.h"
 #include "sp_hash.h"
 #include "sp_sort.h"
@@ -1090,12 +1093,17 @@ static bool conv_bitmap(const GeomDev& g, int64_t n, bool key64) {
           vol <= double(kBitmapCellsPerCandidate) * double(n) * double(g.kv));
 }
 
+// The bitmap is read in 64-cell words; each has the number of set bits before
+// it.  meta: [0] the scan's chunk counter, [32..] the pair counters; the scan's
+// chunk states follow it, so one launch clears both.
+constexpr int kBitmapChunk = 8192;  // 32-bit words a workgroup of the scan covers
 struct BitmapWs {
-  uint32_t* bits;    // [words] occupancy, bit key % 32 of word key / 32
-  uint32_t* prefix;  // [words] set bits in the words before
-  uint32_t* total;   // number of set bits
-  void* scan_ws;
-  int64_t words;
+  uint32_t* bits;     // [words] occupancy, bit key % 32 of word key / 32
+  uint32_t* prefix;   // [words / 2] set bits in the 64-cell words before (written for
+                      // 4 words at a time, and not where all 4 are empty)
+  uint32_t* meta;     // [64]
+  uint64_t* state;    // [chunks]
+  int64_t words, words64, chunks;
 };
 
 template <class W>
@@ -1103,10 +1111,50 @@ static void bitmap_layout(W& w, const GeomDev& g, BitmapWs* out) {
   const int64_t words = cdiv(g.batch * prod_shape(g.out_shape, g.ndim), 32);
   auto* bits = w.template take<uint32_t>(size_t(words));
   auto* prefix = w.template take<uint32_t>(size_t(words));
-  auto* total = w.template take<uint32_t>(64);
-  void* sws = w.template take<char>(scan_workspace_bytes(words));
-  if (out) *out = BitmapWs{bits, prefix, total, sws, words};
+  auto* meta = w.template take<uint32_t>(64);
+  void* state = w.template take<char>(scan_workspace_bytes(words));  // 4 bytes per 4096 words
+  static_assert(kBitmapChunk * 4 >= 8 * kScanChunk, "a chunk's state fits");
+  if (out)
+    *out = BitmapWs{bits, prefix, meta, static_cast<uint64_t*>(state), words, cdiv(words, 2),
+                    cdiv(words, kBitmapChunk)};
 }
+
+// Small pinned host buffers that kernels write their counts to, kept between
+// calls (one per call in flight, whatever the thread or device): a copy of the
+// counts from device memory costs a launch and ~4 us before the host goes on.
+struct PinnedPool {
+  std::mutex m;
+  std::vector<void*> idle;
+};
+static PinnedPool& pinned_pool() {
+  static PinnedPool* p = new PinnedPool;  // (outlives the threads that return buffers to it)
+  return *p;
+}
+class PinnedCounts {
+ public:
+  static constexpr size_t kBytes = 256;
+  int take() {
+    {
+      std::lock_guard<std::mutex> lock(pinned_pool().m);
+      if (!pinned_pool().idle.empty()) {
+        p_ = pinned_pool().idle.back();
+        pinned_pool().idle.pop_back();
+        return SP_OK;
+      }
+    }
+    SP_HIP(hipHostMalloc(&p_, kBytes, hipHostMallocPortable | hipHostMallocMapped));
+    return SP_OK;
+  }
+  ~PinnedCounts() {
+    if (!p_) return;
+    std::lock_guard<std::mutex> lock(pinned_pool().m);
+    pinned_pool().idle.push_back(p_);
+  }
+  uint64_t* data() const { return static_cast<uint64_t*>(p_); }
+
+ private:
+  void* p_ = nullptr;
+};
 
 // Pair counts go to kCountSpread 64-bit counters, one atomic per workgroup on
 // counter blockIdx.x % kCountSpread; the reader sums them (count_sum).  Atomics
@@ -1133,49 +1181,246 @@ static int64_t count_sum(const uint32_t* h) {
   return int64_t(t);
 }
 
-// One thread per input row j: set the bits of its candidate outputs.  The kv
-// candidates of a row come in key order along the fastest dimension, so runs
-// in one word are ORed together before the atomic.
-// The candidates (the table's pairs) are counted into *npairs.
-// (Measured with each row's offsets split over four threads, as conv_fill_bitmap
-// does: 31.5 -> 54.3 us on the LiDAR encoder's first k3 s2 layer, the rows'
-// atomics meeting on the same bitmap words at the same time.)
+// Zeros for the bitmap (16-byte stores; its part of the workspace is padded to
+// 256 bytes) and for the counters and chunk states behind it.
+__global__ __launch_bounds__(256) void bitmap_clear(uint4* __restrict__ bits, int64_t n16,
+                                                    uint32_t* __restrict__ meta, int64_t n_meta) {
+  const int64_t step = int64_t(gridDim.x) * blockDim.x;
+  const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  for (int64_t i = t; i < n16; i += step) bits[i] = make_uint4(0u, 0u, 0u, 0u);
+  for (int64_t i = t; i < n_meta; i += step) meta[i] = 0u;
+}
+
+// Windows of up to 3 offsets in each of up to 3 dimensions (the usual case) are
+// worked out one dimension at a time: at most 9 divisions and bounds tests per
+// row instead of 3 per offset.  A missing leading dimension counts as extent 1.
+static bool win3_ok(const GeomDev& g) {
+  if (g.ndim > 3) return false;
+  for (int d = 0; d < g.ndim; ++d)
+    if (g.ks[d] > 3) return false;
+  return true;
+}
+
+struct Win3 {
+  int32_t o[3][3];  // output coordinate of offset i of dimension d, -1: none
+  int ks[3];
+  uint32_t shape[3];
+};
+
+__device__ __forceinline__ void win3_row(const GeomDev& g, const Coord& c, Win3* w) {
+  const int lead = 3 - g.ndim;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    w->ks[d] = 1;
+    w->shape[d] = 1u;
+#pragma unroll
+    for (int i = 0; i < 3; ++i) w->o[d][i] = i == 0 ? 0 : -1;
+#pragma unroll
+    for (int e = 0; e < 3; ++e) {  // (e = d - lead, as a constant index)
+      if (e != d - lead) continue;
+      w->ks[d] = g.ks[e];
+      w->shape[d] = uint32_t(g.out_shape[e]);
+      const int32_t x = int32_t(c.x[e]);
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        int32_t o;
+        bool ok = c.ok && i < g.ks[e];
+        if (g.mode == SP_PAIR_TRANSPOSE) {
+          o = x * g.st[e] - g.pad[e] + i * g.dil[e];
+        } else {
+          const int32_t num = x + g.pad[e] - i * g.dil[e];
+          const uint32_t q = div31(uint32_t(num >= 0 ? num : 0), g.st_div[e]);
+          ok = ok && num >= 0 && uint32_t(num) == q * uint32_t(g.st[e]);
+          o = int32_t(q);
+        }
+        w->o[d][i] = ok && o >= 0 && o < int32_t(g.out_shape[e]) ? o : -1;
+      }
+    }
+  }
+}
+
+// One thread per input row: set the bits of its candidate outputs, whose number
+// (the table's pairs) goes to *npairs.  Outputs along the fastest dimension that
+// share a word are ORed together first, and a word that already shows them all
+// costs no atomic (a plain read may miss another XCD's bits: one atomic too
+// many).  Bound by the atomics, which go past the XCD's L2: WIN3 takes the
+// valid offsets of each dimension only, at most 2 x 2 x 2 of a k3 s2 window's 27
+// (LiDAR encoder, 4 strided layers: 110 -> 71 us a pass).  (Measured with each
+// row's offsets split over four threads: 31.5 -> 54.3 us on the encoder's first
+// k3 s2 layer, the rows' atomics meeting on the same words at the same time.)
+template <bool WIN3>
 __global__ __launch_bounds__(256) void conv_mark(const int32_t* __restrict__ idx, int64_t n,
-                                                 GeomDev g, uint32_t* __restrict__ bits,
+                                                 GeomDev g, uint32_t* bits,
                                                  unsigned long long* __restrict__ npairs) {
   const int64_t j = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   uint32_t cnt = 0;
+  auto flush = [&](uint32_t w, uint32_t b) {
+    if ((bits[w] & b) != b) atomicOr(&bits[w], b);
+  };
   if (j < n) {
     const Coord c = load_coord(idx, j, g);
-    int off[4] = {0, 0, 0, 0};
     uint32_t cw = 0, cb = 0;  // pending word and its bits (cb == 0: none)
-    for (int k = 0; k < g.kv; ++k) {
-      uint64_t key;
-      if (candidate_key<int32_t>(g, c, off, &key)) {
-        const uint32_t w = uint32_t(key >> 5), b = 1u << uint32_t(key & 31u);
-        if (cb != 0 && w != cw) {
-          atomicOr(&bits[cw], cb);
-          cb = 0;
-        }
-        cw = w;
-        cb |= b;
-        ++cnt;
+    auto add = [&](uint32_t key) {
+      const uint32_t w = key >> 5, b = 1u << (key & 31u);
+      if (cb != 0 && w != cw) {
+        flush(cw, cb);
+        cb = 0;
       }
-      odometer_next(g, off);
+      cw = w;
+      cb |= b;
+      ++cnt;
+    };
+    if constexpr (WIN3) {
+      Win3 w;
+      win3_row(g, c, &w);
+      int m[3];  // each dimension's valid outputs, moved to the front
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        const bool v0 = w.o[d][0] >= 0, v1 = w.o[d][1] >= 0, v2 = w.o[d][2] >= 0;
+        m[d] = int(v0) + int(v1) + int(v2);
+        const int32_t a = v0 ? w.o[d][0] : v1 ? w.o[d][1] : w.o[d][2];
+        const int32_t b = v0 && v1 ? w.o[d][1] : w.o[d][2];
+        w.o[d][0] = a;
+        w.o[d][1] = b;
+      }
+#pragma unroll
+      for (int i = 0; i < 3; ++i) {
+        if (i >= m[0]) break;
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          if (k >= m[1]) break;
+          const uint32_t base =
+              ((uint32_t(c.b) * w.shape[0] + uint32_t(w.o[0][i])) * w.shape[1] +
+               uint32_t(w.o[1][k])) * w.shape[2];
+#pragma unroll
+          for (int l = 0; l < 3; ++l)
+            if (l < m[2]) add(base + uint32_t(w.o[2][l]));
+        }
+      }
+    } else {
+      int off[4] = {0, 0, 0, 0};
+      for (int k = 0; k < g.kv; ++k) {
+        uint64_t key;
+        if (candidate_key<int32_t>(g, c, off, &key)) add(uint32_t(key));
+        odometer_next(g, off);
+      }
     }
-    if (cb != 0) atomicOr(&bits[cw], cb);
+    if (cb != 0) flush(cw, cb);
   }
   block_count(cnt, npairs);
 }
 
-// conv_fill_bitmap splits each input row's kv offsets over the four waves of
-// a workgroup: wave w of workgroup b takes rows 64 b .. 64 b + 63 (one per
-// lane) and the contiguous offsets [w * per, (w + 1) * per), per =
-// ceil(kv / 4).  With one thread walking all kv offsets of its row the launch
-// held too few waves to hide the loop's latency (50k rows: 782 waves on 1 024
-// SIMDs): 26.4 -> 15.2 us on the LiDAR encoder's first k3 s2 layer.
+// Exclusive scan of the 64-cell words' set bits in one launch: a workgroup adds
+// up its chunk, publishes the sum, and its first wave walks back over the
+// chunks before it, 64 at a time, until one knows its own prefix (decoupled
+// look-back: Merrill and Garland, "Single-pass parallel prefix scan with
+// decoupled look-back", 2016).  A chunk's state is one 64-bit word, status in
+// the top bits, so no fence orders it.  Chunks are numbered by a counter as
+// workgroups start, so every chunk waited for belongs to a running workgroup
+// that publishes its sum before it waits itself.  (Sums, their scan and the
+// application as three launches: 20.5 us on the urban k2 s2 table of 134 M
+// output cells, 14.6 a layer on the LiDAR encoder; 14.2 and 5.1 us now.)
+constexpr uint64_t kScanSum = uint64_t(1) << 62, kScanPrefix = uint64_t(2) << 62;
+__global__ __launch_bounds__(512) void bitmap_scan(const uint64_t* __restrict__ bits,
+                                                   int64_t words64, int64_t chunks,
+                                                   uint32_t* __restrict__ prefix, uint64_t* state,
+                                                   uint32_t* meta,
+                                                   const unsigned long long* __restrict__ npairs,
+                                                   uint64_t* __restrict__ result) {
+  constexpr int kPer = kBitmapChunk / 2 / 512;  // 64-cell words per thread
+  __shared__ uint32_t s_scan[9];
+  __shared__ uint32_t s_chunk;
+  __shared__ uint64_t s_base;
+  if (threadIdx.x == 0) s_chunk = atomicAdd(&meta[0], 1u);
+  __syncthreads();
+  const int64_t chunk = s_chunk;
+  if (chunk >= chunks) return;  // (a counter that was not cleared)
+  const int64_t w0 = chunk * (kBitmapChunk / 2) + int64_t(threadIdx.x) * kPer;
+  uint32_t cnt[kPer];
+  uint32_t sum = 0;
+  if (w0 + kPer <= words64) {
+    const ulonglong2* p = reinterpret_cast<const ulonglong2*>(bits + w0);
+#pragma unroll
+    for (int i = 0; i < kPer / 2; ++i) {
+      const ulonglong2 v = p[i];
+      cnt[2 * i] = uint32_t(__popcll(v.x));
+      cnt[2 * i + 1] = uint32_t(__popcll(v.y));
+    }
+  } else {
+#pragma unroll
+    for (int i = 0; i < kPer; ++i)
+      cnt[i] = w0 + i < words64 ? uint32_t(__popcll(bits[w0 + i])) : 0u;
+  }
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) sum += cnt[i];
+  uint32_t tot;
+  uint32_t run = block_exclusive_scan<512>(sum, s_scan, &tot);
+  if (threadIdx.x < 64) {
+    const int lane = int(threadIdx.x);
+    if (lane == 0)
+      __hip_atomic_store(&state[chunk], (chunk == 0 ? kScanPrefix : kScanSum) | tot,
+                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    uint64_t base = 0;
+    for (int64_t top = chunk - 1; top >= 0; top -= 64) {
+      const int64_t at = top - lane;
+      uint64_t v = kScanPrefix;  // (before the first chunk: a prefix of none)
+      for (;;) {
+        if (at >= 0)
+          v = __hip_atomic_load(&state[at], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (!__ballot((v >> 62) == 0)) break;
+        __builtin_amdgcn_s_sleep(1);
+      }
+      const uint64_t known = __ballot((v >> 62) == 2);
+      const int last = known ? __builtin_ctzll(known) : 63;
+      uint64_t part = lane <= last ? v & (kScanSum - 1) : 0;
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) part += __shfl_xor(part, off, 64);
+      base += part;
+      if (known) break;
+    }
+    if (lane == 0) {
+      if (chunk != 0)
+        __hip_atomic_store(&state[chunk], kScanPrefix | (base + tot), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+      s_base = base;
+      if (chunk == chunks - 1) {
+        uint64_t pairs = 0;
+        for (int i = 0; i < kCountSpread; ++i) pairs += npairs[i];
+        result[0] = base + tot;
+        result[1] = pairs;
+      }
+    }
+  }
+  __syncthreads();
+  run += uint32_t(s_base);
+  uint32_t o[kPer];
+#pragma unroll
+  for (int i = 0; i < kPer; ++i) {
+    o[i] = run;
+    run += cnt[i];
+  }
+  if (w0 + kPer <= words64) {
+#pragma unroll
+    for (int i = 0; i < kPer / 4; ++i)
+      if (cnt[4 * i] | cnt[4 * i + 1] | cnt[4 * i + 2] | cnt[4 * i + 3])
+        reinterpret_cast<uint4*>(prefix + w0)[i] =
+            make_uint4(o[4 * i], o[4 * i + 1], o[4 * i + 2], o[4 * i + 3]);
+  } else {
+#pragma unroll
+    for (int i = 0; i < kPer; ++i)
+      if (w0 + i < words64) prefix[w0 + i] = o[i];
+  }
+}
+
+// conv_fill_bitmap splits each input row's kv offsets over the waves of a
+// workgroup, which takes rows 64 b .. 64 b + 63, one per lane.  With one thread
+// walking all kv offsets of its row the launch held too few waves to hide the
+// loop's latency (50k rows: 782 waves on 1 024 SIMDs): 26.4 -> 15.2 us on the
+// LiDAR encoder's first k3 s2 layer.  WIN3: a wave per offset of the leading
+// dimension, its up to 9 lookups in flight together; otherwise four waves, wave
+// w on the contiguous offsets [w * per, (w + 1) * per), per = ceil(kv / 4).
 constexpr int kBitmapRowsPerBlock = 64;
-constexpr int kBitmapParts = 4;  // waves per workgroup, each a part of the offsets
+constexpr int kBitmapParts = 4;
 
 // First offset of this wave's part, its end, and its per-dimension offsets.
 __device__ __forceinline__ void offset_part(const GeomDev& g, int part, int* k0, int* k1,
@@ -1194,21 +1439,34 @@ __device__ __forceinline__ void offset_part(const GeomDev& g, int part, int* k0,
   }
 }
 
-// Output row of a marked key.
-__device__ __forceinline__ int64_t bitmap_rank(const uint32_t* __restrict__ bits,
-                                               const uint32_t* __restrict__ prefix, uint64_t key) {
-  const uint64_t w = key >> 5;
-  const uint32_t below = bits[w] & ((1u << uint32_t(key & 31u)) - 1u);
-  return int64_t(prefix[w]) + __popc(below);
+// Coordinates of a key below 2^31, as an output row [batch, x0, ...] of ndim + 1.
+__device__ __forceinline__ void emit_key(const GeomDev& g, uint32_t key, int32_t* __restrict__ o) {
+  int32_t co[5] = {0, 0, 0, 0, 0};  // the loop is unrolled, so the divisors stay in registers
+#pragma unroll
+  for (int d = 3; d >= 0; --d) {
+    if (d < g.ndim) {
+      const uint32_t q = div31(key, g.out_div[d]);
+      co[d + 1] = int32_t(key - q * uint32_t(g.out_shape[d]));
+      key = q;
+    }
+  }
+  co[0] = int32_t(key);
+#pragma unroll
+  for (int d = 0; d < 5; ++d)
+    if (d <= g.ndim) o[d] = co[d];
 }
 
-// conv_fill with the bitmap's ranks.  The rows' mask words (bit k of word
-// k / 32: offset k has a pair) are gathered from the four parts in the
-// dynamic LDS, mic * 64 words (launched with none when words is null).
+// conv_fill with the bitmap's ranks.  Every pair also writes its output row's
+// coordinates: the pairs of a row write the same values, every kept row has
+// one, and reading the bitmap back for them took longer than all of this
+// (emit: 23 us a layer on the LiDAR encoder).  The rows' mask words (bit k of
+// word k / 32: offset k has a pair) are gathered from the waves in the dynamic
+// LDS, mic * 64 words (launched with none when words is null).
+template <bool WIN3>
 __global__ __launch_bounds__(256) void conv_fill_bitmap(
-    const int32_t* __restrict__ idx, int64_t n, GeomDev g, const uint32_t* __restrict__ bits,
+    const int32_t* __restrict__ idx, int64_t n, GeomDev g, const uint64_t* __restrict__ bits,
     const uint32_t* __restrict__ prefix, int64_t n_keep, int32_t* __restrict__ pf,
-    int32_t* __restrict__ pb, uint32_t* __restrict__ words, int mic) {
+    int32_t* __restrict__ pb, uint32_t* __restrict__ words, int mic, int32_t* __restrict__ out) {
   extern __shared__ uint32_t s_words[];  // [mic][64]
   const int lane = int(threadIdx.x & 63);
   const int64_t j = int64_t(blockIdx.x) * kBitmapRowsPerBlock + lane;
@@ -1217,28 +1475,80 @@ __global__ __launch_bounds__(256) void conv_fill_bitmap(
       s_words[i] = 0u;
     __syncthreads();
   }
+  auto rank_of = [&](uint64_t w, uint32_t before, uint32_t key) -> int64_t {
+    return int64_t(before) + __popcll(w & ((uint64_t(1) << (key & 63u)) - 1u));
+  };
   if (j < n) {
     const Coord c = load_coord(idx, j, g);
-    int off[4], k0, k1;
-    offset_part(g, int(threadIdx.x >> 6), &k0, &k1, off);
-    uint32_t word = 0;
-    for (int k = k0; k < k1; ++k) {
-      uint64_t key;
-      int32_t r = -1;
-      if (candidate_key<int32_t>(g, c, off, &key)) {
-        const int64_t rank = bitmap_rank(bits, prefix, key);
-        r = rank < n_keep ? int32_t(rank) : -1;
+    if constexpr (WIN3) {
+      Win3 w;
+      win3_row(g, c, &w);
+      const int i0 = int(threadIdx.x >> 6);  // (blockDim.x = 64 ks[0] of the 3)
+      const int32_t o0 = i0 == 0 ? w.o[0][0] : i0 == 1 ? w.o[0][1] : w.o[0][2];
+      uint32_t key[9], before[9];
+      uint64_t wd[9];
+      bool ok[9];
+#pragma unroll
+      for (int i1 = 0; i1 < 3; ++i1)
+#pragma unroll
+        for (int i2 = 0; i2 < 3; ++i2) {
+          const int q = i1 * 3 + i2;
+          ok[q] = o0 >= 0 && w.o[1][i1] >= 0 && w.o[2][i2] >= 0;
+          key[q] = ((uint32_t(c.b) * w.shape[0] + uint32_t(o0)) * w.shape[1] +
+                    uint32_t(w.o[1][i1])) * w.shape[2] + uint32_t(w.o[2][i2]);
+          wd[q] = ok[q] ? bits[key[q] >> 6] : 0;
+          before[q] = ok[q] ? prefix[key[q] >> 6] : 0u;
+        }
+      uint32_t word = 0;
+#pragma unroll
+      for (int i1 = 0; i1 < 3; ++i1)
+#pragma unroll
+        for (int i2 = 0; i2 < 3; ++i2) {
+          if (i1 >= w.ks[1] || i2 >= w.ks[2]) continue;
+          const int q = i1 * 3 + i2;
+          const int k = (i0 * w.ks[1] + i1) * w.ks[2] + i2;
+          const int64_t rank = rank_of(wd[q], before[q], key[q]);
+          const int32_t r = ok[q] && rank < n_keep ? int32_t(rank) : -1;
+          if (r >= 0) {
+            if (pf) pf[int64_t(k) * n_keep + r] = int32_t(j);
+            word |= 1u << k;
+            int32_t* o = out + int64_t(r) * (g.ndim + 1);
+            if (g.ndim == 3 && (reinterpret_cast<uintptr_t>(out) & 15u) == 0) {
+              *reinterpret_cast<int4*>(o) = make_int4(int32_t(c.b), o0, w.o[1][i1], w.o[2][i2]);
+            } else {
+              const int32_t co[3] = {o0, w.o[1][i1], w.o[2][i2]};
+              o[0] = int32_t(c.b);
+#pragma unroll
+              for (int d = 0; d < 3; ++d)
+                if (d >= 3 - g.ndim) o[d - (3 - g.ndim) + 1] = co[d];
+            }
+          }
+          if (pb) pb[int64_t(k) * n + j] = r;
+        }
+      if (words && word) atomicOr(&s_words[lane], word);  // (27 offsets: one word)
+    } else {
+      int off[4], k0, k1;
+      offset_part(g, int(threadIdx.x >> 6), &k0, &k1, off);
+      uint32_t word = 0;
+      for (int k = k0; k < k1; ++k) {
+        uint64_t key;
+        int32_t r = -1;
+        if (candidate_key<int32_t>(g, c, off, &key)) {
+          const int64_t rank = rank_of(bits[key >> 6], prefix[key >> 6], uint32_t(key));
+          r = rank < n_keep ? int32_t(rank) : -1;
+        }
+        if (r >= 0) {
+          if (pf) pf[int64_t(k) * n_keep + r] = int32_t(j);
+          word |= 1u << (k & 31);
+          emit_key(g, uint32_t(key), out + int64_t(r) * (g.ndim + 1));
+        }
+        if (pb) pb[int64_t(k) * n + j] = r;
+        if (((k & 31) == 31 || k == k1 - 1) && word) {
+          if (words) atomicOr(&s_words[(k >> 5) * kBitmapRowsPerBlock + lane], word);
+          word = 0;
+        }
+        odometer_next(g, off);
       }
-      if (r >= 0) {
-        if (pf) pf[int64_t(k) * n_keep + r] = int32_t(j);
-        word |= 1u << (k & 31);
-      }
-      if (pb) pb[int64_t(k) * n + j] = r;
-      if (((k & 31) == 31 || k == k1 - 1) && word) {
-        if (words) atomicOr(&s_words[(k >> 5) * kBitmapRowsPerBlock + lane], word);
-        word = 0;
-      }
-      odometer_next(g, off);
     }
   }
   if (words) {
@@ -1247,62 +1557,6 @@ __global__ __launch_bounds__(256) void conv_fill_bitmap(
       const int r = i / mic, w = i % mic;  // row-major: consecutive threads, consecutive words
       const int64_t jr = int64_t(blockIdx.x) * kBitmapRowsPerBlock + r;
       if (jr < n) words[jr * mic + w] = s_words[w * kBitmapRowsPerBlock + r];
-    }
-  }
-}
-
-// Output coordinates of the kept rows: one thread per bitmap word, its set
-// bits in order (rows prefix[w], prefix[w] + 1, ...).
-// Each thread scans 4 words (one 16-byte load; the bitmap sits at the start of
-// a 256-byte aligned workspace part) and reads the prefix of the non-empty
-// ones only: in a sparse volume almost every word is empty, and one thread
-// per word spent the kernel on workgroup dispatch.
-__global__ __launch_bounds__(256) void emit_bitmap_keys(const uint32_t* __restrict__ bits,
-                                                        const uint32_t* __restrict__ prefix,
-                                                        int64_t nwords, GeomDev g, int64_t n_keep,
-                                                        int32_t* __restrict__ out) {
-  const int64_t w0 = (int64_t(blockIdx.x) * blockDim.x + threadIdx.x) * 4;
-  if (w0 >= nwords) return;
-  uint32_t m4[4];
-  if (w0 + 4 <= nwords) {
-    const uint4 v = *reinterpret_cast<const uint4*>(bits + w0);
-    m4[0] = v.x;
-    m4[1] = v.y;
-    m4[2] = v.z;
-    m4[3] = v.w;
-  } else {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) m4[i] = w0 + i < nwords ? bits[w0 + i] : 0u;
-  }
-  if ((m4[0] | m4[1] | m4[2] | m4[3]) == 0) return;
-  for (int i = 0; i < 4; ++i) {
-    uint32_t m = m4[i];
-    if (m == 0) continue;
-    const int64_t w = w0 + i;
-    int64_t r = prefix[w];
-    while (m != 0 && r < n_keep) {
-      const int b = __ffs(m) - 1;
-      m &= m - 1u;
-      uint32_t rem = uint32_t(w) * 32u + uint32_t(b);  // bitmap keys are below 2^31
-      int32_t co[5] = {0, 0, 0, 0, 0};  // (batch, x0, .., x3); the loop is unrolled, so the
-#pragma unroll                          // divisors stay in registers across rows
-      for (int d = 3; d >= 0; --d) {
-        if (d < g.ndim) {
-          const uint32_t q = div31(rem, g.out_div[d]);  // rem < 2^31
-          co[d + 1] = int32_t(rem - q * uint32_t(g.out_shape[d]));
-          rem = q;
-        }
-      }
-      co[0] = int32_t(rem);
-      int32_t* o = out + r * (g.ndim + 1);
-      if (g.ndim == 3 && (reinterpret_cast<uintptr_t>(out) & 15u) == 0) {  // one 16-byte store
-        *reinterpret_cast<int4*>(o) = make_int4(co[0], co[1], co[2], co[3]);
-      } else {
-#pragma unroll
-        for (int d = 0; d < 5; ++d)
-          if (d <= g.ndim) o[d] = co[d];
-      }
-      ++r;
     }
   }
 }
@@ -1706,23 +1960,27 @@ int sp_pairgen_conv_build(const sp_geom* g, const int32_t* indices, int64_t n, v
   if (conv_bitmap(d, n, key64)) {
     BitmapWs b;
     bitmap_layout(c, d, &b);
-    const int64_t fb = cdiv(cdiv(b.words, 4), 256);
-    fill_i32x4<<<unsigned(fb < 4096 ? fb : 4096), 256, 0, s>>>(
-        reinterpret_cast<int32_t*>(b.bits), b.words, 0);
-    SP_LAUNCHED();
-    // total[0]: set bits (from the scan); total[32..63]: the pair counters
-    auto* npairs = reinterpret_cast<unsigned long long*>(b.total + 32);
-    SP_HIP(hipMemsetAsync(npairs, 0, kCountSpread * sizeof(unsigned long long), s));
-    conv_mark<<<unsigned(cdiv(n, 256)), 256, 0, s>>>(indices, n, d, b.bits, npairs);
-    SP_LAUNCHED();
-    SP_CHECK_ARG(cdiv(b.words, 256) <= kMaxGridX, "pairgen: output volume too large");
-    rc = exclusive_scan_popc(b.bits, b.prefix, b.words, b.total, b.scan_ws, s);
+    PinnedCounts counts;
+    rc = counts.take();
     if (rc) return rc;
-    uint32_t h[32 + 2 * kCountSpread] = {};
-    SP_HIP(hipMemcpyAsync(h, b.total, sizeof(h), hipMemcpyDeviceToHost, s));
+    const int64_t n16 = cdiv(b.words, 4), fb = cdiv(n16, 256);
+    const int64_t n_meta = (reinterpret_cast<char*>(b.state + b.chunks) -
+                            reinterpret_cast<char*>(b.meta)) / int64_t(sizeof(uint32_t));
+    SP_CHECK_ARG(b.chunks <= kMaxGridX, "pairgen: output volume too large");
+    bitmap_clear<<<unsigned(fb < 4096 ? fb : 4096), 256, 0, s>>>(
+        reinterpret_cast<uint4*>(b.bits), n16, b.meta, n_meta);
+    SP_LAUNCHED();
+    auto* npairs = reinterpret_cast<unsigned long long*>(b.meta + 32);
+    auto mark = win3_ok(d) ? conv_mark<true> : conv_mark<false>;
+    mark<<<unsigned(cdiv(n, 256)), 256, 0, s>>>(indices, n, d, b.bits, npairs);
+    SP_LAUNCHED();
+    bitmap_scan<<<unsigned(b.chunks), 512, 0, s>>>(reinterpret_cast<const uint64_t*>(b.bits),
+                                                   b.words64, b.chunks, b.prefix, b.state, b.meta,
+                                                   npairs, counts.data());
+    SP_LAUNCHED();
     SP_HIP(hipStreamSynchronize(s));
-    *n_out = int64_t(h[0]);
-    if (n_pairs) *n_pairs = count_sum(h + 32);
+    *n_out = int64_t(counts.data()[0]);
+    if (n_pairs) *n_pairs = int64_t(counts.data()[1]);
     return SP_OK;
   }
   ConvWs w;
@@ -1817,11 +2075,18 @@ int sp_pairgen_conv_fill(const sp_geom* g, const int32_t* indices, int64_t n, co
     BitmapWs b;
     bitmap_layout(c, d, &b);
     const size_t lds = mask_words_bwd ? size_t(mic) * kBitmapRowsPerBlock * 4 : 0;  // <= 32 KiB
-    conv_fill_bitmap<<<unsigned(cdiv(n, kBitmapRowsPerBlock)), 256, lds, s>>>(
-        indices, n, d, b.bits, b.prefix, n_keep, pair_fwd, pair_bwd, mask_words_bwd, mic);
-    SP_LAUNCHED();
-    emit_bitmap_keys<<<unsigned(cdiv(b.words, 1024)), 256, 0, s>>>(b.bits, b.prefix, b.words, d,
-                                                                   n_keep, out_indices);
+    const auto* bits64 = reinterpret_cast<const uint64_t*>(b.bits);
+    const unsigned blocks64 = unsigned(cdiv(n, kBitmapRowsPerBlock));
+    if (win3_ok(d)) {
+      const unsigned threads = 64u * unsigned(d.ndim == 3 ? d.ks[0] : 1);
+      conv_fill_bitmap<true><<<blocks64, threads, lds, s>>>(indices, n, d, bits64, b.prefix, n_keep,
+                                                            pair_fwd, pair_bwd, mask_words_bwd,
+                                                            mic, out_indices);
+    } else {
+      conv_fill_bitmap<false><<<blocks64, 64 * kBitmapParts, lds, s>>>(
+          indices, n, d, bits64, b.prefix, n_keep, pair_fwd, pair_bwd, mask_words_bwd, mic,
+          out_indices);
+    }
     SP_LAUNCHED();
     return SP_OK;
   }
