@@ -132,6 +132,8 @@ _SIGNATURES = {
     "sp_wgrad_workspace_size": (_SZ, [_I64, _I64, _I64, _I64]),
     "sp_conv_wgrad": (ctypes.c_int, [_P, _I64, _P, _I64, _I32, _I64, _I64, _I64, _P, _P, _P,
                                      _I64, _P, _P, _SZ, _P]),
+    "sp_batchnorm_eval": (ctypes.c_int, [_P, _I32, _I64, _I64, _P, _P, _P, _P, _I32,
+                                         ctypes.c_float, _I32, _P, _P]),
     "sp_maxpool_fwd": (ctypes.c_int, [_P, _I32, _I64, _I64, _P, _I64, _I64, _P, _P]),
     "sp_maxpool_bwd": (ctypes.c_int, [_P, _P, _P, _I32, _I64, _I64, _P, _I64, _I64, _P, _P]),
     "sp_avgpool_fwd": (ctypes.c_int, [_P, _I32, _I64, _I64, _P, _I64, _I64, _P, _P, _P]),

@@ -18,6 +18,8 @@ from collections import OrderedDict
 import torch
 from torch import nn
 
+from spconv_triton.pytorch._impl import norm as _norm
+
 
 def _sparse_tensor_cls():
     from spconv_triton.pytorch.core import SparseConvTensor
@@ -79,11 +81,22 @@ class SparseSequential(SparseModule):
 
     def forward(self, x):
         sct = _sparse_tensor_cls()
-        for module in self._modules.values():
+        mods = list(self._modules.values())
+        i = 0
+        while i < len(mods):
+            module = mods[i]
+            i += 1
             if is_spconv_module(module):
                 x = module(x)
             elif isinstance(x, sct):
                 if x.indices.shape[0] != 0:
+                    if (type(module) is nn.BatchNorm1d and _norm.passes_unobserved()
+                            and _norm.fusable_bn(module, x.features)):
+                        # an inference pass's plain BatchNorm1d, with the plain ReLU after it
+                        relu = i < len(mods) and _norm.fusable_relu(mods[i])
+                        i += relu
+                        x = x.replace_feature(_norm.batchnorm_eval(module, x.features, relu))
+                        continue
                     x = x.replace_feature(module(x.features))
             else:
                 x = module(x)

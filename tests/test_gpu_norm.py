@@ -1,0 +1,118 @@
+"""Eval BatchNorm1d (+ ReLU) inside SparseSequential: the one-launch kernel against
+fp64 and against torch's modules, and the modules it must leave to torch."""
+
+import numpy as np
+import pytest
+import torch
+from torch import nn
+
+pytestmark = pytest.mark.gpu
+
+DEV = "cuda:0"
+F16, BF16, F32 = torch.float16, torch.bfloat16, torch.float32
+UNIT = {F16: 2.0 ** -11, BF16: 2.0 ** -8, F32: 2.0 ** -24}
+
+
+def _tensor(feats):
+    import spconv_triton.pytorch as spconv
+
+    n = feats.shape[0]
+    idx = np.stack([np.zeros(n), np.arange(n) // 64 // 64, np.arange(n) // 64 % 64,
+                    np.arange(n) % 64], 1).astype(np.int32)
+    return spconv.SparseConvTensor(feats, torch.from_numpy(idx).to(DEV), [64, 64, 64], 1)
+
+
+def _bn(C, dtype, affine=True, seed=0):
+    g = torch.Generator().manual_seed(seed)
+    bn = nn.BatchNorm1d(C, affine=affine)
+    with torch.no_grad():
+        bn.running_mean.copy_(torch.randn(C, generator=g))
+        bn.running_var.copy_(torch.rand(C, generator=g) * 2 + 0.01)
+        if affine:
+            bn.weight.copy_(torch.randn(C, generator=g))
+            bn.bias.copy_(torch.randn(C, generator=g))
+    return bn.to(DEV).to(dtype).eval()
+
+
+@pytest.mark.parametrize("rows,C,dtype,pdtype,affine,relu", [
+    (1, 16, F16, F16, True, True), (4097, 32, F16, F16, True, True),
+    (255, 2048, F16, F32, True, False), (255, 2056, F16, F16, True, True),  # past 256 pieces
+    (1000, 20, F16, F16, True, True), (513, 3, F16, F16, True, False),  # no whole vectors
+    (777, 48, BF16, BF16, True, True), (777, 64, BF16, F32, False, True),
+    (4097, 64, F32, F32, True, True), (33, 5, F32, F32, False, False)])
+def test_batchnorm_eval_matches_fp64(rows, C, dtype, pdtype, affine, relu):
+    """|error| <= 1 rounding of the result's type + 8 fp32 roundings of the terms."""
+    import spconv_triton.pytorch as spconv
+
+    torch.manual_seed(rows + C)
+    x = torch.randn(rows, C, device=DEV).to(dtype)
+    bn = _bn(C, pdtype, affine)
+    net = spconv.SparseSequential(bn, *([nn.ReLU()] if relu else []))
+    with torch.no_grad():
+        y = net(_tensor(x)).features
+        t = bn(x)
+        t = torch.relu(t) if relu else t
+    m, v = bn.running_mean.double(), bn.running_var.double()
+    w = bn.weight.double() if affine else torch.ones_like(m)
+    b = bn.bias.double() if affine else torch.zeros_like(m)
+    scale = w / torch.sqrt(v + bn.eps)
+    ref = (x.double() - m) * scale + b
+    mag = (x.double().abs() + m.abs()) * scale.abs() + b.abs()
+    ref = ref.clamp(min=0) if relu else ref
+    bound = UNIT[dtype] * ref.abs() + 8 * 2.0 ** -24 * mag + (2.0 ** -25 if dtype is F16 else 0)
+    assert y.dtype == dtype and ((y.double() - ref).abs() <= bound).all()
+    assert ((y.double() - t.double()).abs() <= 2 * bound).all()
+
+
+def test_batchnorm_special_values():
+    import spconv_triton.pytorch as spconv
+
+    x = torch.randn(64, 16, device=DEV).half()
+    x[3, 2], x[4, 5], x[5, 7] = float("nan"), float("inf"), -float("inf")
+    bn = _bn(16, F16)
+    with torch.no_grad():
+        y = spconv.SparseSequential(bn, nn.ReLU())(_tensor(x)).features
+        t = torch.relu(bn(x))
+    assert torch.equal(torch.isnan(y), torch.isnan(t)) and torch.isnan(y[3, 2])
+    assert torch.equal(torch.isinf(y), torch.isinf(t))
+
+
+class _MyBN(nn.BatchNorm1d):
+    def forward(self, x):
+        return super().forward(x) + 1
+
+
+def test_observed_modules_run_themselves(monkeypatch):
+    """Hooks, subclasses, replaced forwards, training mode and gradients keep torch's modules."""
+    import spconv_triton.pytorch as spconv
+    from spconv_triton.pytorch._impl import norm
+
+    calls = []
+    real = norm.batchnorm_eval
+    monkeypatch.setattr(norm, "batchnorm_eval",
+                        lambda *a: (calls.append(1), real(*a))[1])
+    x = torch.randn(100, 16, device=DEV)
+    bn, relu = _bn(16, F32), nn.ReLU()
+    net = spconv.SparseSequential(bn, relu)
+    with torch.no_grad():
+        net(_tensor(x))
+        assert len(calls) == 1
+        for mod in (bn, relu):  # a hook on either is called
+            seen = []
+            h = mod.register_forward_hook(lambda m, i, o: seen.append(o))
+            y = net(_tensor(x)).features
+            h.remove()
+            assert len(seen) == 1 and torch.equal(seen[0].clamp(min=0), y)
+        assert len(calls) == 2  # the ReLU's hook left the BatchNorm fusable
+        relu.forward = lambda v: v * 2
+        assert torch.equal(net(_tensor(x)).features, real(bn, x, False) * 2)
+        del relu.forward
+        my = _MyBN(16).to(DEV).eval()
+        my.load_state_dict(bn.state_dict())
+        n = len(calls)
+        torch.testing.assert_close(spconv.SparseSequential(my)(_tensor(x)).features, bn(x) + 1)
+        spconv.SparseSequential(bn.train())(_tensor(x))
+        bn.eval()
+        assert len(calls) == n
+    y = net(_tensor(x.clone().requires_grad_(True))).features
+    assert y.requires_grad and len(calls) == n
