@@ -361,13 +361,23 @@ __global__ __launch_bounds__(256) void wgrad_partial(
       }
   };
 
-  floatx16 acc[MT][MT];
+  // fp32: each stage's sum is made by itself and added to the share's, so that
+  // no chain of fp32 sums is longer than a stage's pairs or a share's stages
+  // (75k surface rows, 349k pairs, 64 -> 64: 2.2e-7 of the result from fp64, with
+  // one chain per share 5.0e-7 and, at twice the shares, 3.6e-7)
+  constexpr bool STAGED = sizeof(T) == 4;
+  floatx16 acc[MT][MT], sum[STAGED ? MT : 1][STAGED ? MT : 1];
+  auto zero = [](floatx16& v) {
+#pragma unroll
+    for (int i = 0; i < 16; ++i) v[i] = 0.f;
+  };
 #pragma unroll
   for (int a = 0; a < MT; ++a)
 #pragma unroll
-    for (int b = 0; b < MT; ++b)
-#pragma unroll
-      for (int i = 0; i < 16; ++i) acc[a][b][i] = 0.f;
+    for (int b = 0; b < MT; ++b) {
+      zero(acc[a][b]);
+      if constexpr (STAGED) zero(sum[a][b]);
+    }
 
   int32_t iv[2], ov[2], iv2[2], ov2[2];
   frag xv[2][NV], gv[2][NV];
@@ -400,6 +410,21 @@ __global__ __launch_bounds__(256) void wgrad_partial(
 #pragma unroll
         for (int mn = 0; mn < MT; ++mn) MF::mma(a[mc], b[mn], acc[mc][mn]);
     }
+    if constexpr (STAGED) {
+#pragma unroll
+      for (int mc = 0; mc < MT; ++mc)
+#pragma unroll
+        for (int mn = 0; mn < MT; ++mn) {
+          sum[mc][mn] += acc[mc][mn];
+          zero(acc[mc][mn]);
+        }
+    }
+  }
+  if constexpr (STAGED) {
+#pragma unroll
+    for (int mc = 0; mc < MT; ++mc)
+#pragma unroll
+      for (int mn = 0; mn < MT; ++mn) acc[mc][mn] = sum[mc][mn];
   }
   // D[c][n]: lane holds column n = l32 of rows c = 8*(i/4) + 4*h + (i%4)
   float* ps = part + int64_t(slot) * K * C;
@@ -899,18 +924,17 @@ static int wgrad_block(int64_t C, int64_t K) { return C >= 128 && K >= 128 ? 128
 
 // Shares a call aims at, and the slots its partials need: an offset's last
 // share may be a short one, so there are at most kv more shares than aimed at.
-// fp32 results take 64 shares per offset (at least 512 workgroups in all), so
-// that no chain of fp32 sums is long; for 16-bit ones, whose rounding hides
-// that, the fewest that fill the chip: every share writes and reads a fp32
-// partial of its block.  Measured (us a call, 256 / 512 / 768 / 1024 / 1536 /
+// The fewest that fill the chip: every share writes and reads a fp32 partial of
+// its block.  Split-bf16 operands, whose fp32 results are summed in one chain a
+// share, take at least 64 workgroups per offset, so that none is long.  Measured (us a call, 256 / 512 / 768 / 1024 / 1536 /
 // 2048 workgroups): urban 240k rows, 410k pairs, 64 -> 64 33.2 / 30.5 / 33.8 /
 // 35.4 / 37.1 / 42.4; k2 s2 64 -> 128 33.2 / 27.8 / 28.6 / 29.9 / 32.2 / 36.6;
 // 75k rows, 349k pairs, 256 -> 128 (128-wide blocks) 108 / 107 / 100 / 99 /
 // 108 / 117, 256 -> 256 189 / 183 / 165 / 166 / 166 / 176.
-static int wgrad_target(int64_t kv, int64_t C, int64_t K, int64_t n_rows, bool f32) {
+static int wgrad_target(int64_t kv, int64_t C, int64_t K, int64_t n_rows, bool split) {
   const int bw = wgrad_block(C, K);
   int64_t wgs = bw == 128 ? 1024 : 512;
-  if (f32 && wgs < 64 * kv) wgs = 64 * kv;
+  if (split && wgs < 64 * kv) wgs = 64 * kv;
   int64_t t = cdiv(wgs, cdiv(C, bw) * cdiv(K, bw));
   const int64_t by_len = cdiv(n_rows * kv, 128);  // a stage of pairs each, if every entry were one
   if (t > by_len) t = by_len;
@@ -919,8 +943,8 @@ static int wgrad_target(int64_t kv, int64_t C, int64_t K, int64_t n_rows, bool f
 // Blocks up to this many values an offset are reduced by 16 waves a workgroup
 // (few workgroups, and a dense offset has most of the shares), larger ones by 4.
 constexpr int64_t kWgWideReduce = 8192;
-static int64_t wgrad_slots(int64_t kv, int64_t C, int64_t K, int64_t n_rows, bool f32) {
-  return wgrad_target(kv, C, K, n_rows, f32) + kv;
+static int64_t wgrad_slots(int64_t kv, int64_t C, int64_t K, int64_t n_rows, bool split) {
+  return wgrad_target(kv, C, K, n_rows, split) + kv;
 }
 
 // ---- the forward without a caller workspace (sp_conv_fwd_noalloc) ---------
@@ -1071,9 +1095,8 @@ int sp_conv_wgrad(const void* x, int64_t n_in, const void* g, int64_t n_out, int
   SP_CHECK_ARG(Kg * Cg < (int64_t(1) << 30) && row_stride < (int64_t(1) << 31),
                "wgrad: weight or table too large");
   const int elem = split ? SP_BF16 : dtype;
-  const bool f32 = split || elem == SP_F32;
-  const int64_t slots = wgrad_slots(kv, Cg, Kg, row_stride, f32);
-  const int target = wgrad_target(kv, Cg, Kg, row_stride, f32);
+  const int64_t slots = wgrad_slots(kv, Cg, Kg, row_stride, split);
+  const int target = wgrad_target(kv, Cg, Kg, row_stride, split);
   const size_t need = sp_wgrad_workspace_size(Kg, kv, Cg, row_stride);
   if (!ws || ws_bytes < need)
     return set_error(SP_ERR_WORKSPACE, "wgrad: workspace %zu < %zu", ws_bytes, need);
