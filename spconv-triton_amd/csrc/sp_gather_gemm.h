@@ -885,6 +885,248 @@ __global__ __launch_bounds__(256, 2) void gather_gemm_direct(
 }
 
 // ---------------------------------------------------------------------------
+// narrow kernel: the direct path for outputs of at most 32 columns
+// ---------------------------------------------------------------------------
+// direct_tile's 64 x 64 waves would spend half their MFMAs, weight loads and
+// accumulators on columns that do not exist; 64 rows x 32 columns take 106
+// registers, so four workgroups fit on a CU instead of two and hide the gathers
+// for each other.  Same items and summation order: results are bit-identical.
+// Bound by the gathers' latency: two steps in flight and four workgroups a CU
+// measured as well as three or four steps and three.  Measured without a gather
+// plan (us, direct -> narrow, and the staged kernel without its plan's build,
+// ~25 us a table; fp16 unless said): LiDAR encoder 80k rows 4 -> 16 30.7 -> 14.4
+// (22.7), 193k rows 16 -> 32 38.2 -> 15.9 (22.0), 32 -> 32 40.2 -> 27.0 (27.7);
+// 80k rows fp32 48 -> 20 137 -> 70 (130); 2 000 rows fp32 16 -> 16 24.7 -> 14.  Two
+// such blocks for 64 columns gather every row twice: slower than direct_tile
+// (metric layer 80 -> 85, urban 64 -> 64 54 -> 62).
+
+// ROWB: what a row is a whole number of: 16-byte pieces, 8-byte halves of them, or
+// elements (0).  KS: K-steps of an item; 1 for rows of at most 2 V elements,
+// whose second step would multiply zeros (skipped: sums stay the same).
+template <typename T, typename OutT, int ROWB, int KS>
+__global__ __launch_bounds__(256, ROWB == 0 && KS == 2 ? 3 : 4) void gather_gemm_narrow(
+    const T* __restrict__ A, const T* __restrict__ Bt, const int32_t* __restrict__ pairs,
+    const float* __restrict__ bias, OutT* __restrict__ out, GemmBufs nb, int64_t n_src, int64_t M,
+    int N, int R, int Rp, int kv) {
+  using frag = typename Mfma<T>::frag;
+  constexpr int V = Mfma<T>::V;
+  constexpr uint32_t ES = sizeof(T);
+  constexpr int kChunk = kChunkBytes / int(ES);
+  constexpr int DEPTH = 2;  // steps of A rows and weights in flight
+  // row-contiguous loads through an LDS slot, as in direct_tile (whole chunks only)
+  constexpr bool SLOT = ROWB == 16 && sizeof(T) == 2 && KS == 2;
+  // fp32 MFMAs take 8 x as long a product: those of a 32-row block without a pair are skipped
+  constexpr bool SKIP = sizeof(T) == 4;
+  extern __shared__ __align__(16) unsigned char smem[];
+  const int64_t tile = xcd_tile(blockIdx.x, gridDim.x);
+
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int h = lane >> 5, l32 = lane & 31;
+  const int64_t slot0 = tile * kTileRows + wave * 64;
+  const int64_t my_row = slot0 + lane;
+  const bool row_ok = my_row < M;
+
+  const __amdgpu_buffer_rsrc_t ra = make_rsrc(A, nb.a_bytes);
+  const __amdgpu_buffer_rsrc_t rb = make_rsrc(Bt, nb.bt_bytes);
+  const __amdgpu_buffer_rsrc_t ro = make_rsrc(out, nb.out_bytes);
+  const __amdgpu_buffer_rsrc_t rp = make_rsrc(pairs, nb.pairs_bytes);
+
+  const int G = kv < kGroupOffsets ? kv : kGroupOffsets;
+  const int E = G + kPad;
+  const DirectLds L = direct_lds(E, uint32_t(sizeof(OutT)));
+  uint32_t* s_kb = reinterpret_cast<uint32_t*>(smem + L.kb_off) + wave * E;
+  uint32_t* s_src = reinterpret_cast<uint32_t*>(smem + L.src_off) + wave * E * 64;
+  unsigned char* aslot = smem + L.a_off + uint32_t(wave) * 2048u;
+
+  const uint32_t row_bytes = uint32_t(R) * ES;
+  const uint32_t slab_bytes = uint32_t(N) * V * ES;
+  const uint32_t k_bytes = uint32_t(Rp / V) * slab_bytes;
+  const int nrc = Rp / kChunk;
+  const int col = l32;
+  const uint32_t bcol = col < N ? uint32_t(col) * V * ES : kColOob;
+
+  floatx16 acc[2];
+#pragma unroll
+  for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+    for (int i = 0; i < 16; ++i) acc[mt][i] = 0.f;
+  for (int kc = 0; kc < kv; kc += G) {
+    const int kn = kv - kc < G ? kv - kc : G;
+    int nact = 0;
+    constexpr int kTabBatch = 14;
+    for (int u0 = 0; u0 < kn; u0 += kTabBatch) {
+      int32_t v[kTabBatch];
+#pragma unroll
+      for (int u = 0; u < kTabBatch; ++u) {
+        const bool in = row_ok && u0 + u < kn;
+        const int64_t e = int64_t(kc + u0 + u) * M + my_row;
+        v[u] = int32_t(__builtin_amdgcn_raw_buffer_load_b32(rp, in ? uint32_t(e * 4) : kOob, 0, 0));
+      }
+#pragma unroll
+      for (int u = 0; u < kTabBatch; ++u) {
+        const bool ok = row_ok && u0 + u < kn && v[u] >= 0 && v[u] < n_src;
+        if (u0 + u < kn && __ballot(ok)) {  // wave-uniform
+          s_src[(nact * 32 + l32) * 2 + h] = ok ? uint32_t(v[u]) * row_bytes : kOob;
+          if (lane == 0) s_kb[nact] = uint32_t(kc + u0 + u) * k_bytes;
+          ++nact;
+        }
+      }
+    }
+    // one padding item: no source row, out-of-range B
+    s_src[(nact * 32 + l32) * 2 + h] = kOob;
+    if (lane == 0) s_kb[nact] = kBOob;
+    nact = __builtin_amdgcn_readfirstlane(nact);
+    if (nact == 0) continue;
+
+    struct Cur {
+      int rc, it;
+    };
+    // the next step: items of a chunk, then the next chunk's, then the padding item
+    auto advance = [&](Cur& c) {
+      if (c.it < nact && ++c.it == nact && c.rc + 1 < nrc) {
+        c.it = 0;
+        ++c.rc;
+      }
+    };
+    uint32_t bl[KS];
+#pragma unroll
+    for (int ks = 0; ks < KS; ++ks) bl[ks] = bcol + uint32_t(ks * 2 + h) * slab_bytes;
+    const uint32_t chunk_b = 4u * slab_bytes;
+    auto load_b = [&](const Cur& c, frag (&b)[KS]) {
+      const uint32_t kr = s_kb[c.it] + uint32_t(c.rc) * chunk_b;
+#pragma unroll
+      for (int ks = 0; ks < KS; ++ks) b[ks] = buf_frag<T>(rb, kr + bl[ks]);
+    };
+    const int rsub = lane >> 2, pc = lane & 3;
+    auto load_a = [&](const Cur& c, frag (&a)[KS][2], uint32_t& live) {
+      if constexpr (SLOT) {
+        const uint2 r0 = *reinterpret_cast<const uint2*>(s_src + (c.it * 32 + rsub) * 2);
+        const uint2 r1 = *reinterpret_cast<const uint2*>(s_src + (c.it * 32 + 16 + rsub) * 2);
+        const uint32_t b4[2][2] = {{r0.x, r0.y}, {r1.x, r1.y}};
+        const int e0 = c.rc * kChunk + pc * V;
+#pragma unroll
+        for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+          for (int mt = 0; mt < 2; ++mt)
+            a[ks][mt] = buf_frag<T>(
+                ra, (b4[ks][mt] != kOob && e0 < R) ? b4[ks][mt] + uint32_t(e0) * ES : kOob);
+      } else {
+        const uint2 e = *reinterpret_cast<const uint2*>(s_src + (c.it * 32 + l32) * 2);
+        const uint32_t s2[2] = {e.x, e.y};
+        if constexpr (SKIP) live = (__ballot(e.x != kOob) ? 1u : 0u) | (__ballot(e.y != kOob) ? 2u : 0u);
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks) {
+          const int e0 = c.rc * kChunk + (ks * 2 + h) * V;
+#pragma unroll
+          for (int mt = 0; mt < 2; ++mt) {
+            const uint32_t at = s2[mt] + uint32_t(e0) * ES;
+            if constexpr (ROWB == 16) {
+              a[ks][mt] = buf_frag<T>(ra, (s2[mt] != kOob && e0 < R) ? at : kOob);
+            } else if constexpr (ROWB == 8) {
+              using u32x2 = __attribute__((ext_vector_type(2))) uint32_t;
+              using u32x4 = __attribute__((ext_vector_type(4))) uint32_t;
+              const u32x2 lo = __builtin_amdgcn_raw_buffer_load_b64(
+                  ra, (s2[mt] != kOob && e0 < R) ? at : kOob, 0, 0);
+              const u32x2 hi = __builtin_amdgcn_raw_buffer_load_b64(
+                  ra, (s2[mt] != kOob && e0 + V / 2 < R) ? at + 8u : kOob, 0, 0);
+              a[ks][mt] = __builtin_bit_cast(frag, u32x4{lo[0], lo[1], hi[0], hi[1]});
+            } else {
+              a[ks][mt] = buf_frag_elems<T>(ra, s2[mt], e0, R);
+            }
+          }
+        }
+      }
+    };
+    const uint32_t wr_row = chunk_base(uint32_t(rsub)) ^ uint32_t(pc << 4);
+    const uint32_t rd_row = chunk_base(uint32_t(l32));
+    auto mma = [&](frag (&a)[KS][2], const frag (&b)[KS], uint32_t live) {
+      if constexpr (SLOT) {
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt) {
+#pragma unroll
+          for (int ks = 0; ks < 2; ++ks)
+            *reinterpret_cast<frag*>(aslot + wr_row + uint32_t(ks) * 1024u) = a[ks][mt];
+#pragma unroll
+          for (int ks = 0; ks < 2; ++ks)
+            a[ks][mt] = *reinterpret_cast<const frag*>(aslot +
+                                                       (rd_row ^ uint32_t((ks * 2 + h) << 4)));
+        }
+      }
+      if constexpr (SKIP) {
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+          if (live & (1u << mt)) {  // wave-uniform
+#pragma unroll
+            for (int ks = 0; ks < KS; ++ks) Mfma<T>::mma(a[ks][mt], b[ks], acc[mt]);
+          }
+      } else {
+#pragma unroll
+        for (int ks = 0; ks < KS; ++ks)
+#pragma unroll
+          for (int mt = 0; mt < 2; ++mt) Mfma<T>::mma(a[ks][mt], b[ks], acc[mt]);
+      }
+    };
+    frag a[DEPTH][KS][2], b[DEPTH][KS];
+    uint32_t live[DEPTH];
+    Cur cur{0, 0};
+#pragma unroll
+    for (int d = 0; d < DEPTH; ++d) {
+      load_b(cur, b[d]);
+      load_a(cur, a[d], live[d]);
+      advance(cur);
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    const int n_steps = nrc * nact;  // (steps past it read the padding item)
+    for (int j = 0; j < n_steps; j += DEPTH) {
+#pragma unroll
+      for (int d = 0; d < DEPTH; ++d) {
+        mma(a[d], b[d], live[d]);
+        __builtin_amdgcn_sched_barrier(0);
+        load_b(cur, b[d]);
+        load_a(cur, a[d], live[d]);
+        advance(cur);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    }
+  }
+  __syncthreads();  // the tables are free for the epilogue
+  constexpr uint32_t OS = sizeof(OutT);
+  constexpr uint32_t pitch = 32u * OS + 16u;
+  constexpr int kPer16 = int(16 / OS);
+  unsigned char* stage = smem + L.src_off + uint32_t(wave) * 32u * pitch;
+  const float bv = (bias && col < N) ? bias[col] : 0.f;
+  const bool whole = N % kPer16 == 0;
+#pragma unroll
+  for (int mt = 0; mt < 2; ++mt) {
+    if (whole) {
+#pragma unroll
+      for (int i = 0; i < 16; ++i)
+        *reinterpret_cast<OutT*>(stage + uint32_t(8 * (i / 4) + 4 * h + (i % 4)) * pitch +
+                                 uint32_t(l32) * OS) = from_f32<OutT>(acc[mt][i] + bv);
+      constexpr int kPieces = 32 / kPer16;
+      constexpr int kRows = 64 / kPieces;
+      const int p = lane % kPieces, pr = lane / kPieces, c = p * kPer16;
+#pragma unroll
+      for (int j = 0; j < 32 / kRows; ++j) {
+        const int lr = pr + j * kRows;
+        const uint4 v = *reinterpret_cast<const uint4*>(stage + uint32_t(lr) * pitch + uint32_t(p) * 16u);
+        const int64_t row = slot0 + mt * 32 + lr;
+        const uint32_t off = (row < M && c < N) ? uint32_t((row * N + c) * int64_t(OS)) : kOob;
+        __builtin_amdgcn_raw_buffer_store_b128(
+            __builtin_bit_cast(__attribute__((ext_vector_type(4))) uint32_t, v), ro, off, 0, 0);
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < 16; ++i) {
+        const int64_t row = slot0 + mt * 32 + 8 * (i / 4) + 4 * h + (i % 4);
+        const uint32_t off = (row < M && col < N) ? uint32_t((row * N + col) * int64_t(OS)) : kOob;
+        buf_store<OutT>(from_f32<OutT>(acc[mt][i] + bv), ro, off);
+      }
+    }
+  }
+}
+
+// ---------------------------------------------------------------------------
 // staged kernel
 // ---------------------------------------------------------------------------
 

@@ -682,6 +682,31 @@ static int launch_direct(dim3 grid, hipStream_t s, const T* A, const T* bt, cons
   return SP_OK;
 }
 
+template <typename T, typename OutT>
+static int launch_narrow(hipStream_t s, const T* A, const T* bt, const int32_t* pairs, OutT* o,
+                         GemmBufs nb, const GemmCall& c) {
+  constexpr int V = Mfma<T>::V;
+  const int G = c.kv < kGroupOffsets ? c.kv : kGroupOffsets;
+  const uint32_t lds = direct_lds(G + kPad, uint32_t(sizeof(OutT))).total;
+  using Kern = decltype(&gather_gemm_narrow<T, OutT, 16, 2>);
+  constexpr Kern kerns[3][2] = {
+      {gather_gemm_narrow<T, OutT, 16, 1>, gather_gemm_narrow<T, OutT, 16, 2>},
+      {gather_gemm_narrow<T, OutT, 8, 1>, gather_gemm_narrow<T, OutT, 8, 2>},
+      {gather_gemm_narrow<T, OutT, 0, 1>, gather_gemm_narrow<T, OutT, 0, 2>}};
+  const bool halves = int64_t(c.R) * int64_t(sizeof(T)) % 8 == 0 &&
+                      reinterpret_cast<uintptr_t>(A) % 8 == 0;
+  const int row = c.vec ? 0 : halves ? 1 : 2, ks = c.R <= 2 * V ? 0 : 1;
+  static bool attr_set[3][2] = {};  // per kernel instance
+  int rc = allow_lds(reinterpret_cast<const void*>(kerns[row][ks]),
+                     direct_lds(kGroupOffsets + kPad, uint32_t(sizeof(OutT))).total,
+                     attr_set[row][ks]);
+  if (rc) return rc;
+  kerns[row][ks]<<<dim3(unsigned(cdiv(c.M, kTileRows))), 256, lds, s>>>(
+      A, bt, pairs, c.bias, o, nb, c.n_src, c.M, c.N, c.R, c.Rp, c.kv);
+  SP_LAUNCHED();
+  return SP_OK;
+}
+
 // LDS of the staged kernel: its own layout, or the direct path's for an
 // overflow tile (smaller for every kv the plans cover; the max keeps it safe).
 static uint32_t staged_kernel_lds(int E, int kv, uint32_t out_size) {
@@ -827,6 +852,11 @@ static int launch_gemm_typed(const T* A, const T* bt, const int32_t* pairs, void
   GemmBufs nb{uint32_t(a_bytes), uint32_t(bt_bytes), uint32_t(p_bytes), uint32_t(o_bytes)};
   const unsigned gy = unsigned(cdiv(c.N, 64));
   OutT* o = static_cast<OutT*>(out);
+  // outputs of at most 32 columns without a plan or an order: the narrow kernel
+  // (the output types the modules ask for; others take the direct kernel)
+  if constexpr (std::is_same<T, OutT>::value || std::is_same<OutT, float>::value) {
+    if (!c.planned && !c.order && c.N <= 32) return launch_narrow<T, OutT>(s, A, bt, pairs, o, nb, c);
+  }
   if (c.vec) return launch_modes<T, OutT, true>(unsigned(gx), gy, s, A, bt, pairs, o, nb, c);
   return launch_modes<T, OutT, false>(unsigned(gx), gy, s, A, bt, pairs, o, nb, c);
 }
