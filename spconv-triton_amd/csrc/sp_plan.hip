@@ -37,9 +37,13 @@ __global__ __launch_bounds__(kPlanThreads) void plan_build_kernel(
     int32_t* __restrict__ count, int32_t* __restrict__ rows_out, int32_t* __restrict__ nact_out,
     int32_t* __restrict__ koff_out, uint16_t* __restrict__ addr_out, int E,
     const uint32_t* __restrict__ words, int mic) {
-  // sort path: the entries; bitmap path: NP / 2 bitmap words, then NP / 2
-  // word rank offsets
-  __shared__ int32_t keys[NP];
+  // sort path: the entries; bitmap path: kBmWords bitmap words, then as many
+  // word rank offsets.  The bitmap takes windows of 131072 rows also where a
+  // tile has few entries: sized by the entries alone (16384 rows at kv 8) the
+  // few wide tiles of an upsampling table, sorted, were most of its build
+  // (8 x 240k table 27.8 -> 10.0 us); 32 KB of LDS still leave a CU full.
+  constexpr int kKeys = NP < 8192 ? 8192 : NP;
+  __shared__ int32_t keys[kKeys];
   __shared__ uint32_t scan_lds[kPlanThreads / 64 + 1];
   // dense: item number of offset k in the tile, or -1; COMPACT: offset of item i
   __shared__ int32_t s_item[kPlanMaxItems];
@@ -51,7 +55,7 @@ __global__ __launch_bounds__(kPlanThreads) void plan_build_kernel(
                 "one wave numbers the items");
   static_assert(!COMPACT || NP >= kTileRows * kPlanMaxItems, "a tile's entries fit in NP");
   constexpr int32_t kNone = 0x7fffffff;
-  constexpr int kBmWords = NP / 2;
+  constexpr int kBmWords = kKeys / 2;
   const int tid = threadIdx.x;
   const int64_t tile = blockIdx.x;
   const int64_t r0 = tile * kTileRows;
@@ -137,30 +141,41 @@ __global__ __launch_bounds__(kPlanThreads) void plan_build_kernel(
     }
   }
   const int n_ent = kTileRows * (COMPACT ? s_nact : kv);
-  // ---- entries into registers; window and items
+  // ---- entries into registers; window and items.  All of a thread's loads are
+  // issued before any entry is looked at: with the item flags set in LDS
+  // between them each load waited for the one before (27 x 240k urban table
+  // 25.9 -> 17.0 us, 27 x 200k surface table 26.9 -> 19.2).
   int32_t v[PER];
-  int32_t lo = kNone, hi = -1;
+  const uint64_t live =
+      COMPACT ? 0 : uint64_t(s_live[0]) | (uint64_t(s_live[1]) << 32);  // (kv <= 64)
+  constexpr int kStep = kPlanThreads / kTileRows;  // offsets (items) side by side
+  const int wq = __builtin_amdgcn_readfirstlane(tid / kTileRows), lr0 = tid & (kTileRows - 1);
+  const bool row_ok = r0 + lr0 < M;
 #pragma unroll
   for (int i = 0; i < PER; ++i) {
-    const int e = i * kPlanThreads + tid;
-    int32_t key = kNone;
-    if (e < n_ent) {
-      const int q = e / kTileRows;  // dense: the offset; COMPACT: the item
-      const int k = COMPACT ? s_item[q] : q;
-      const int64_t r = r0 + (e - q * kTileRows);
-      if (r < M && (COMPACT || ((s_live[k >> 5] >> (k & 31)) & 1u))) {
-        const int32_t x = pairs[int64_t(k) * M + r];
-        if (x >= 0 && x < n_src) {
-          key = x;
-          if (!COMPACT) s_item[k] = 0;  // every writer stores the same value
-        }
-      }
+    const int q = i * kStep + wq;  // dense: the offset; COMPACT: the item (wave-uniform)
+    const bool in = q * kTileRows < n_ent && (COMPACT || ((live >> (q & 63)) & 1u));
+    const int k = COMPACT ? __builtin_amdgcn_readfirstlane(in ? s_item[q] : 0) : q;
+    const int32_t* col = pairs + int64_t(k) * M + r0;
+    v[i] = in && row_ok ? col[lr0] : -1;
+  }
+  int32_t lo = kNone, hi = -1;
+  uint64_t seen = 0;  // dense: offsets of this thread's valid entries
+#pragma unroll
+  for (int i = 0; i < PER; ++i) {
+    const int32_t x = v[i];
+    const bool ok = x >= 0 && x < n_src;
+    if (ok) {
+      lo = x < lo ? x : lo;
+      hi = x > hi ? x : hi;
+      if (!COMPACT) seen |= uint64_t(1) << ((i * kStep + wq) & 63);
     }
-    v[i] = key;
-    if (key != kNone) {
-      lo = key < lo ? key : lo;
-      hi = key > hi ? key : hi;
-    }
+    v[i] = ok ? x : kNone;
+  }
+  if (!COMPACT) {  // lane l marks offset l for the wave
+    uint32_t s0 = wave_or(uint32_t(seen)), s1 = wave_or(uint32_t(seen >> 32));
+    const int l = tid & 63;
+    if (((l < 32 ? s0 : s1) >> (l & 31)) & 1u) s_item[l] = 0;  // every writer stores the same value
   }
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) {
@@ -216,17 +231,20 @@ __global__ __launch_bounds__(kPlanThreads) void plan_build_kernel(
     U = int(total);
     for (int w = w0; w < w1; ++w) {
       pre[w] = pos;
-      uint32_t bits = bm[w];
-      if (U < kLdsRows)
+      pos += uint32_t(__builtin_popcount(bm[w]));
+    }
+    __syncthreads();
+    // the list, a word per thread at a time: a tile's own rows fill consecutive
+    // words, which one thread would write bit by bit
+    if (U < kLdsRows)
+      for (int w = tid; w < nw; w += kPlanThreads) {
+        uint32_t bits = bm[w], at = pre[w];
         while (bits) {
           const int b = __builtin_ctz(bits);
           bits &= bits - 1;
-          rows_t[pos++] = lo + w * 32 + b;
+          rows_t[at++] = lo + w * 32 + b;
         }
-      else
-        pos += uint32_t(__builtin_popcount(bits));
-    }
-    __syncthreads();
+      }
   } else {
 #pragma unroll
     for (int i = 0; i < PER; ++i) keys[i * kPlanThreads + tid] = v[i];

@@ -172,6 +172,23 @@ def test_plan_matches_numpy(case):
         assert n_over == 0
 
 
+@pytest.mark.parametrize("kv", [1, 2, 8, 27])
+@pytest.mark.parametrize("span", [16385, 131072, 131073])
+def test_plan_wide_windows(kv, span):
+    """Few entries over a wide window of source rows: at the last window that
+    the bitmap takes (131072 rows, also where a tile has few entries), one past
+    it, and one past what the tile's entries alone would size it for."""
+    rng = np.random.default_rng(kv * 7 + span)
+    M, n_src, lo = TILE + 37, 200_000, 1234
+    pf = np.full((kv, M), -1, dtype=np.int32)
+    for r in range(M):
+        for k in rng.choice(kv, size=min(kv, 3), replace=False):
+            pf[k, r] = lo + rng.integers(0, span)
+    for r in (0, TILE):  # both ends of the window in each tile
+        pf[0, r], pf[0, r + 1] = lo, lo + span - 1
+    _check_plan(torch.from_numpy(pf).to(DEV), n_src)
+
+
 @pytest.mark.parametrize("kv", [27, 64, 81, 125])
 def test_plan_with_row_words_identical(kv):
     """A plan built with the rows' mask words (the build reads only the offsets
