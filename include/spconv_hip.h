@@ -427,7 +427,8 @@ size_t sp_point2voxel_workspace_size(int64_t n_points, int64_t max_voxels);
  * its mean, utils.py:145-152), indices [max_voxels, ndim] int32 in ZYX order,
  * num_per_voxel [max_voxels] int32 (clamped counts), pc_voxel_id [n_points]
  * int64 (voxel of every point, -1 when dropped) and *num_voxels.  Blocks the
- * host once, to read the voxel count. */
+ * host once, to read the voxel count; what is enqueued after that runs on in
+ * the stream, as every call's work does. */
 int sp_point2voxel(const void* points, int32_t dtype, int64_t n_points, int64_t point_cols,
                    int32_t ndim, const double* vsize_xyz, const double* coors_min_xyz,
                    const int64_t* grid_size_xyz, int32_t num_point_features, int64_t max_voxels,

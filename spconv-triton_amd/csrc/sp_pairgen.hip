@@ -23,11 +23,10 @@
 //    is written back into its hash slot as its output row.
 #include <type_traits>
 
-#include <mutex>
-#include <vector>
 
 #include "sp_common.h"
 #include "sp_hash.h"
+#include "sp_lookback.h"
 #include "sp_sort.h"
 
 namespace sp {
@@ -1119,43 +1118,6 @@ static void bitmap_layout(W& w, const GeomDev& g, BitmapWs* out) {
                     cdiv(words, kBitmapChunk)};
 }
 
-// Small pinned host buffers that kernels write their counts to, kept between
-// calls (one per call in flight, whatever the thread or device): a copy of the
-// counts from device memory costs a launch and ~4 us before the host goes on.
-struct PinnedPool {
-  std::mutex m;
-  std::vector<void*> idle;
-};
-static PinnedPool& pinned_pool() {
-  static PinnedPool* p = new PinnedPool;  // (outlives the threads that return buffers to it)
-  return *p;
-}
-class PinnedCounts {
- public:
-  static constexpr size_t kBytes = 256;
-  int take() {
-    {
-      std::lock_guard<std::mutex> lock(pinned_pool().m);
-      if (!pinned_pool().idle.empty()) {
-        p_ = pinned_pool().idle.back();
-        pinned_pool().idle.pop_back();
-        return SP_OK;
-      }
-    }
-    SP_HIP(hipHostMalloc(&p_, kBytes, hipHostMallocPortable | hipHostMallocMapped));
-    return SP_OK;
-  }
-  ~PinnedCounts() {
-    if (!p_) return;
-    std::lock_guard<std::mutex> lock(pinned_pool().m);
-    pinned_pool().idle.push_back(p_);
-  }
-  uint64_t* data() const { return static_cast<uint64_t*>(p_); }
-
- private:
-  void* p_ = nullptr;
-};
-
 // Pair counts go to kCountSpread 64-bit counters, one atomic per workgroup on
 // counter blockIdx.x % kCountSpread; the reader sums them (count_sum).  Atomics
 // on one address serialise: one per wave onto a single counter took ~25 us of
@@ -1311,16 +1273,10 @@ __global__ __launch_bounds__(256) void conv_mark(const int32_t* __restrict__ idx
 }
 
 // Exclusive scan of the 64-cell words' set bits in one launch: a workgroup adds
-// up its chunk, publishes the sum, and its first wave walks back over the
-// chunks before it, 64 at a time, until one knows its own prefix (decoupled
-// look-back: Merrill and Garland, "Single-pass parallel prefix scan with
-// decoupled look-back", 2016).  A chunk's state is one 64-bit word, status in
-// the top bits, so no fence orders it.  Chunks are numbered by a counter as
-// workgroups start, so every chunk waited for belongs to a running workgroup
-// that publishes its sum before it waits itself.  (Sums, their scan and the
-// application as three launches: 20.5 us on the urban k2 s2 table of 134 M
-// output cells, 14.6 a layer on the LiDAR encoder; 14.2 and 5.1 us now.)
-constexpr uint64_t kScanSum = uint64_t(1) << 62, kScanPrefix = uint64_t(2) << 62;
+// up its chunk and gets the sum of the chunks before it by look-back.  (Sums,
+// their scan and the application as three launches: 20.5 us on the urban k2 s2
+// table of 134 M output cells, 14.6 a layer on the LiDAR encoder; 14.2 and 5.1
+// us now.)
 __global__ __launch_bounds__(512) void bitmap_scan(const uint64_t* __restrict__ bits,
                                                    int64_t words64, int64_t chunks,
                                                    uint32_t* __restrict__ prefix, uint64_t* state,
@@ -1360,24 +1316,7 @@ __global__ __launch_bounds__(512) void bitmap_scan(const uint64_t* __restrict__ 
     if (lane == 0)
       __hip_atomic_store(&state[chunk], (chunk == 0 ? kScanPrefix : kScanSum) | tot,
                          __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-    uint64_t base = 0;
-    for (int64_t top = chunk - 1; top >= 0; top -= 64) {
-      const int64_t at = top - lane;
-      uint64_t v = kScanPrefix;  // (before the first chunk: a prefix of none)
-      for (;;) {
-        if (at >= 0)
-          v = __hip_atomic_load(&state[at], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        if (!__ballot((v >> 62) == 0)) break;
-        __builtin_amdgcn_s_sleep(1);
-      }
-      const uint64_t known = __ballot((v >> 62) == 2);
-      const int last = known ? __builtin_ctzll(known) : 63;
-      uint64_t part = lane <= last ? v & (kScanSum - 1) : 0;
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) part += __shfl_xor(part, off, 64);
-      base += part;
-      if (known) break;
-    }
+    const uint64_t base = scan_lookback(state, chunk, lane);
     if (lane == 0) {
       if (chunk != 0)
         __hip_atomic_store(&state[chunk], kScanPrefix | (base + tot), __ATOMIC_RELAXED,

@@ -6,24 +6,27 @@
 // stores up to max_num_points_per_voxel points per voxel in arrival order,
 // with torch.unique, scatter_reduce, argsort and cumsum.  Here:
 //   1. insert: every in-range point's linear voxel key goes into an
-//      open-addressing hash (sp_hash.h) with the point index as value; the
-//      table keeps the smallest index, i.e. the voxel's first point;
-//   2. first: a point is "first" when the table holds its own index; an
-//      exclusive scan over the first flags, in point order, numbers the
-//      voxels in order of first occurrence (the FCFS ids), and the ids are
-//      written back into the table;
-//   3. assign: every point reads its voxel id; points of voxels past the cap
-//      get -1; per-voxel point counts by atomic adds (order-free);
-//   4. a stable radix sort of the kept points by voxel id keeps arrival order
-//      inside every voxel; an exclusive scan of the counts gives each voxel's
-//      first position, so a point's slot is its sorted position minus that;
-//   5. scatter: points with slot < max_points_per_voxel are copied into their
-//      voxel; per voxel the clamped count and the coordinates (decoded from
-//      the key of its first point, ZYX order) are written.
-// The only host synchronisation is the final read of the voxel count, which
-// sizes the returned views (the reference reads it too: uniq.numel()).
+//      open-addressing hash (sp_hash.h).  A slot keeps the smallest point index
+//      (the voxel's first point) and counts its points; a point keeps its slot
+//      and the count it met, a place of its own in the voxel's list;
+//   2. number: a point is "first" when its slot holds its own index.  One scan
+//      over the points, of first points and of their voxels' counts, numbers
+//      the voxels in order of first occurrence (the FCFS ids) and says where
+//      each one's list starts; the first point writes its voxel's clamped count
+//      and coordinates (decoded from the key, ZYX order);
+//   3. place: every point reads its voxel id (-1 past the cap) and enters
+//      itself in its voxel's list, at the place it got from the insertion;
+//   4. rank: a list is in no order, but a point's slot is the number of smaller
+//      indices in it; points with slot < max_points_per_voxel are copied there.
+// Step 4 reads a voxel's list once for each of its points, so where a voxel has
+// too many points (p2v_rank_max) steps 3 and 4 are a stable radix sort of the points
+// by voxel id instead (arrival order inside every voxel).
+// The only host synchronisation is the read of the voxel count after step 2: it
+// sizes the returned views (the reference reads it too: uniq.numel()), and the
+// flag that comes with it chooses step 4.
 #include "sp_common.h"
 #include "sp_hash.h"
+#include "sp_lookback.h"
 #include "sp_sort.h"
 
 namespace sp {
@@ -35,10 +38,69 @@ struct P2VGeom {
   int64_t gsize[4];
 };
 
+// A voxel of the hash, in one 16-byte slot.  The insertion is bound by its three
+// atomics a point, which go past the XCD's L2 (200k points: 31
+// us; with a plain read first, that spares the CAS or the minimum where it
+// shows the key or a smaller index, 32).
+struct alignas(16) P2VSlot {
+  uint64_t key;
+  int32_t first;   // the smallest point index
+  uint32_t count;  // its points; after the numbering its id
+};
+// Voxels of up to this many points are ranked by their lists (p2v_rank), which
+// reads a voxel's list once per point, or about 3 maxpts of it where that is
+// less; past about 16M reads the sort is the faster.  Whole calls, lists and
+// sort, us: 200k points, 64 a voxel, all kept 128 and 140; 250 a voxel, 5 kept
+// 134 and 152; 250, all kept 198 and 153; 1M points, 64 a voxel, all kept 459
+// and 346; 250, 32 kept 422 and 318; 250, 8 kept 330 and 309.
+static uint32_t p2v_rank_max(int64_t n, int maxpts) {
+  const int64_t reads = (int64_t(1) << 24) / n;  // a point
+  if (3 * int64_t(maxpts) <= reads) return 256u;
+  return uint32_t(reads < 8 ? 8 : reads > 256 ? 256 : reads);
+}
+// counters in the workspace: scan chunks handed out, "a voxel has more than
+// rank_max points", "the table is full"
+enum { kMetaChunk = 0, kMetaLong = 16, kMetaOverflow = 17, kMetaWords = 64 };
+struct P2VTable {
+  P2VSlot* slots;
+  uint64_t mask;
+  uint32_t* overflow;
+
+  // The slot of `key`, inserted when absent; -1 (and the overflow flag) when
+  // the table is full.
+  __device__ int64_t insert(uint64_t key) const {
+    uint64_t s = mix64(key) & mask;
+    for (uint64_t i = 0; i <= mask; ++i) {
+      const uint64_t prev = atomicCAS((unsigned long long*)&slots[s].key,
+                                      (unsigned long long)kEmpty64, (unsigned long long)key);
+      if (prev == kEmpty64 || prev == key) return int64_t(s);
+      s = (s + 1) & mask;
+    }
+    atomicExch(overflow, 1u);
+    return -1;
+  }
+};
+
+// The table, the counters and the voxels (n_vox floats), in one launch.
+__global__ __launch_bounds__(256) void p2v_clear(uint4* __restrict__ slots, int64_t n_slots,
+                                                 uint32_t* __restrict__ meta, int64_t n_meta,
+                                                 float* __restrict__ voxels, int64_t n_vox) {
+  const int64_t step = int64_t(gridDim.x) * blockDim.x;
+  const int64_t t0 = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
+  const uint4 none = make_uint4(0u, 0u, 0u, 0u);
+  static_assert(kEmpty64 == ~uint64_t(0) && sizeof(P2VSlot) == 16, "an empty key is all ones");
+  for (int64_t i = t0; i < n_slots; i += step) slots[i] = make_uint4(~0u, ~0u, 0x7fffffffu, 0u);
+  for (int64_t i = t0; i < n_meta; i += step) meta[i] = 0u;
+  const int64_t n4 = (reinterpret_cast<uintptr_t>(voxels) & 15) == 0 ? n_vox / 4 : 0;
+  for (int64_t i = t0; i < n4; i += step) reinterpret_cast<uint4*>(voxels)[i] = none;
+  for (int64_t i = 4 * n4 + t0; i < n_vox; i += step) voxels[i] = 0.f;
+}
+
 template <typename F>
 __global__ __launch_bounds__(256) void p2v_insert(const F* __restrict__ pc, int64_t n,
-                                                  int64_t cols, P2VGeom g, Table64 t,
-                                                  int64_t* __restrict__ keys) {
+                                                  int64_t cols, P2VGeom g, P2VTable t,
+                                                  uint32_t rank_max, uint32_t* meta, int64_t* __restrict__ slot,
+                                                  uint32_t* __restrict__ place) {
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= n) return;
   bool ok = true;
@@ -50,39 +112,147 @@ __global__ __launch_bounds__(256) void p2v_insert(const F* __restrict__ pc, int6
     ok = ok && q >= F(0) && q < F(g.gsize[d]);
     lin = lin * g.gsize[d] + (ok ? int64_t(q) : 0);
   }
-  keys[i] = ok ? lin : -1;
-  if (ok) t.insert(uint64_t(lin), int32_t(i));
+  int64_t s = -1;
+  if (ok) s = t.insert(uint64_t(lin));
+  if (s >= 0) {
+    const uint32_t before = atomicAdd(&t.slots[s].count, 1u);
+    atomicMin(&t.slots[s].first, int32_t(i));
+    place[i] = before;
+    if (before == rank_max) meta[kMetaLong] = 1u;
+  }
+  slot[i] = s;
 }
 
-__global__ __launch_bounds__(256) void p2v_first(const int64_t* __restrict__ keys, int64_t n,
-                                                 Table64 t, uint32_t* __restrict__ first) {
+// kNumThreads * kNumPer points a workgroup; the sums of the chunks before it by
+// look-back, voxels in the low 31 bits of a state and points above them (both
+// below 2^31).  A slot's count becomes the voxel's id: only its first point
+// reads the count.  The last chunk's workgroup writes the totals to host
+// memory: result[0] voxels, [1] whether one has more than rank_max points, [2]
+// the table's overflow flag.
+// Each chunk costs one atomic on the chunk counter, and these serialise: 391
+// chunks of 512 points took 35 us (200k points, three atomics each), 196 of 1024
+// with one each 15.3, 98 of 2048 19.0 (too few workgroups).
+constexpr int kNumThreads = 512, kNumPer = 2, kNumChunk = kNumThreads * kNumPer;
+__global__ __launch_bounds__(kNumThreads) void p2v_number(
+    const int64_t* __restrict__ slot, int64_t n, int64_t chunks, P2VTable t, int64_t max_vox,
+    int maxpts, P2VGeom g, uint32_t* __restrict__ counts,
+    uint32_t* __restrict__ start, int32_t* __restrict__ npv, int32_t* __restrict__ indices,
+    uint64_t* state, uint32_t* meta, uint64_t* __restrict__ result) {
+  __shared__ uint32_t s_scan[2][kNumThreads / 64 + 1];
+  __shared__ uint32_t s_chunk;
+  __shared__ uint64_t s_base;
+  if (threadIdx.x == 0) s_chunk = atomicAdd(&meta[kMetaChunk], 1u);
+  __syncthreads();
+  const int64_t chunk = s_chunk;
+  if (chunk >= chunks) return;  // (a counter that was not cleared)
+  const int64_t i0 = chunk * kNumChunk + int64_t(threadIdx.x) * kNumPer;
+  int64_t sl[kNumPer];
+  uint32_t c[kNumPer];
+#pragma unroll
+  for (int j = 0; j < kNumPer; ++j) sl[j] = i0 + j < n ? slot[i0 + j] : -1;
+#pragma unroll
+  for (int j = 0; j < kNumPer; ++j)
+    c[j] = sl[j] >= 0 && t.slots[sl[j]].first == int32_t(i0 + j) ? t.slots[sl[j]].count : 0u;
+  uint32_t nf = 0, np = 0;
+#pragma unroll
+  for (int j = 0; j < kNumPer; ++j) {
+    nf += c[j] != 0u ? 1u : 0u;
+    np += c[j];
+  }
+  uint32_t tot_f, tot_p;
+  uint32_t vid = block_exclusive_scan<kNumThreads>(nf, s_scan[0], &tot_f);
+  uint32_t at = block_exclusive_scan<kNumThreads>(np, s_scan[1], &tot_p);
+  const uint64_t tot = uint64_t(tot_f) | (uint64_t(tot_p) << 31);
+  if (threadIdx.x < 64) {
+    const int lane = int(threadIdx.x);
+    if (lane == 0)
+      __hip_atomic_store(&state[chunk], (chunk == 0 ? kScanPrefix : kScanSum) | tot,
+                         __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    const uint64_t base = scan_lookback(state, chunk, lane);
+    if (lane == 0) {
+      if (chunk != 0)
+        __hip_atomic_store(&state[chunk], kScanPrefix | (base + tot), __ATOMIC_RELAXED,
+                           __HIP_MEMORY_SCOPE_AGENT);
+      s_base = base;
+      if (chunk == chunks - 1) {
+        result[0] = (base + tot) & 0x7fffffffu;
+        result[1] = meta[kMetaLong];
+        result[2] = meta[kMetaOverflow];
+      }
+    }
+  }
+  __syncthreads();
+  vid += uint32_t(s_base & 0x7fffffffu);
+  at += uint32_t(s_base >> 31);
+#pragma unroll
+  for (int j = 0; j < kNumPer; ++j) {
+    if (c[j] == 0u) continue;
+    t.slots[sl[j]].count = vid;
+    if (int64_t(vid) < max_vox) {
+      counts[vid] = c[j];
+      start[vid] = at;
+      npv[vid] = int32_t(c[j] < uint32_t(maxpts) ? c[j] : uint32_t(maxpts));
+      uint64_t key = t.slots[sl[j]].key;
+      for (int d = g.ndim - 1; d >= 0; --d) {
+        // (a 64-bit division takes several times a 32-bit one's instructions)
+        const uint64_t size = uint64_t(g.gsize[d]);
+        const uint64_t q = (key | size) >> 32 ? key / size : uint32_t(key) / uint32_t(size);
+        indices[int64_t(vid) * g.ndim + (g.ndim - 1 - d)] = int32_t(key - q * size);  // ZYX
+        key = q;
+      }
+    }
+    ++vid;
+    at += c[j];
+  }
+}
+
+// Lists (list != null) or, for the sort, a key per point; pc_voxel_id either
+// way.  place_vid[i], the point's place, becomes its voxel, or max_vox (dropped
+// points sort last).
+__global__ __launch_bounds__(256) void p2v_place(const int64_t* __restrict__ slot, int64_t n,
+                                                 const P2VSlot* __restrict__ slots,
+                                                 int64_t max_vox,
+                                                 const uint32_t* __restrict__ start,
+                                                 uint32_t* place_vid,
+                                                 int64_t* __restrict__ pc_voxel_id,
+                                                 uint32_t* __restrict__ list) {
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const int64_t k = keys[i];
-  first[i] = (k >= 0 && t.find(uint64_t(k)) == int32_t(i)) ? 1u : 0u;
+  const int64_t s = slot[i];
+  const uint32_t v = s >= 0 ? slots[s].count : 0u;
+  const bool kept = s >= 0 && int64_t(v) < max_vox;
+  pc_voxel_id[i] = kept ? int64_t(v) : -1;
+  if (kept && list) list[start[v] + place_vid[i]] = uint32_t(i);
+  place_vid[i] = kept ? v : uint32_t(max_vox);
 }
 
-__global__ __launch_bounds__(256) void p2v_set_ids(const int64_t* __restrict__ keys, int64_t n,
-                                                   Table64 t, const uint32_t* __restrict__ first,
-                                                   const uint32_t* __restrict__ rank) {
-  const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  if (i >= n || !first[i]) return;
-  t.set_value(t.find_slot(uint64_t(keys[i])), int32_t(rank[i]));
-}
-
-__global__ __launch_bounds__(256) void p2v_assign(const int64_t* __restrict__ keys, int64_t n,
-                                                  Table64 t, int64_t max_vox,
-                                                  int64_t* __restrict__ pc_voxel_id,
-                                                  uint32_t* __restrict__ sort_key,
-                                                  uint32_t* __restrict__ counts) {
+// A point's slot: the smaller indices in its voxel's list, eight loads in
+// flight, until there are maxpts of them.
+template <typename F>
+__global__ __launch_bounds__(256) void p2v_rank(const F* __restrict__ pc, int64_t n, int64_t cols,
+                                                int nfeat, const uint32_t* __restrict__ vid,
+                                                const uint32_t* __restrict__ counts,
+                                                const uint32_t* __restrict__ start,
+                                                const uint32_t* __restrict__ list,
+                                                int64_t max_vox, int maxpts,
+                                                float* __restrict__ voxels) {
   const int64_t i = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
   if (i >= n) return;
-  const int64_t k = keys[i];
-  const int32_t vid = k >= 0 ? t.find(uint64_t(k)) : -1;
-  const bool kept = vid >= 0 && vid < max_vox;
-  pc_voxel_id[i] = kept ? int64_t(vid) : -1;
-  sort_key[i] = kept ? uint32_t(vid) : uint32_t(max_vox);  // dropped points sort last
-  if (kept) atomicAdd(&counts[vid], 1u);
+  const uint32_t v = vid[i];
+  if (int64_t(v) >= max_vox) return;
+  const uint32_t c = counts[v];
+  const uint32_t* l = list + start[v];
+  uint32_t r = 0;
+  for (uint32_t j = 0; c > 1u && j < c && r < uint32_t(maxpts); j += 8) {
+    uint32_t x[8];
+#pragma unroll
+    for (uint32_t u = 0; u < 8; ++u) x[u] = l[j + u < c ? j + u : c - 1u];
+#pragma unroll
+    for (uint32_t u = 0; u < 8; ++u) r += j + u < c && x[u] < uint32_t(i) ? 1u : 0u;
+  }
+  if (r >= uint32_t(maxpts)) return;
+  float* dst = voxels + (int64_t(v) * maxpts + r) * nfeat;
+  for (int f = 0; f < nfeat; ++f) dst[f] = float(pc[i * cols + f]);
 }
 
 template <typename F>
@@ -101,31 +271,12 @@ __global__ __launch_bounds__(256) void p2v_scatter(
   for (int f = 0; f < nfeat; ++f) dst[f] = float(pc[int64_t(i) * cols + f]);
 }
 
-__global__ __launch_bounds__(256) void p2v_voxels(
-    const uint32_t* __restrict__ counts, const uint32_t* __restrict__ start,
-    const uint32_t* __restrict__ perm, const int64_t* __restrict__ keys,
-    const uint32_t* __restrict__ n_unique, int64_t max_vox, int maxpts, P2VGeom g,
-    int32_t* __restrict__ npv, int32_t* __restrict__ indices) {
-  const int64_t v = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int64_t nv = int64_t(*n_unique) < max_vox ? int64_t(*n_unique) : max_vox;
-  if (v >= nv) return;
-  const uint32_t c = counts[v];
-  npv[v] = int32_t(c < uint32_t(maxpts) ? c : uint32_t(maxpts));
-  int64_t key = keys[perm[start[v]]];  // the voxel's first point
-  for (int d = g.ndim - 1; d >= 0; --d) {
-    indices[v * g.ndim + (g.ndim - 1 - d)] = int32_t(key % g.gsize[d]);  // ZYX order
-    key /= g.gsize[d];
-  }
-}
-
 // Empty slots of every voxel get the mean over all max_points_per_voxel slots
 // divided by the point count (reference utils.py:145-152), summed in slot order.
 __global__ __launch_bounds__(256) void p2v_empty_mean(float* __restrict__ voxels,
                                                       const int32_t* __restrict__ npv,
-                                                      const uint32_t* __restrict__ n_unique,
-                                                      int64_t max_vox, int maxpts, int nfeat) {
+                                                      int64_t nv, int maxpts, int nfeat) {
   const int64_t t = int64_t(blockIdx.x) * blockDim.x + threadIdx.x;
-  const int64_t nv = int64_t(*n_unique) < max_vox ? int64_t(*n_unique) : max_vox;
   if (t >= nv * nfeat) return;
   const int64_t v = t / nfeat;
   const int f = int(t % nfeat);
@@ -138,51 +289,41 @@ __global__ __launch_bounds__(256) void p2v_empty_mean(float* __restrict__ voxels
 }
 
 struct P2VWs {
-  int64_t* keys;
-  uint32_t* first;
-  uint32_t* rank;
-  uint32_t* sort_key;
+  int64_t* slot;
+  uint32_t* place;  // then vid
   uint32_t* counts;
   uint32_t* start;
-  uint32_t* n_unique;
-  uint64_t* tkeys;
-  int32_t* tvals;
-  int* overflow;
-  void* sort_ws;
-  void* scan_ws;
+  uint32_t* meta;
+  uint64_t* state;
+  P2VSlot* slots;
+  void* sort_ws;  // the voxels' lists, or the sort's
   uint64_t cap;
+  int64_t chunks;
 };
 
 template <class W>
 static void p2v_layout(W& w, int64_t n, int64_t max_vox, P2VWs* out) {
   uint64_t cap = 1024;
   while (cap < uint64_t(n) * 2) cap <<= 1;
-  const int64_t scan_len = n > max_vox ? n : max_vox;
-  auto* keys = w.template take<int64_t>(size_t(n));
-  auto* first = w.template take<uint32_t>(size_t(n));
-  auto* rank = w.template take<uint32_t>(size_t(n));
-  auto* sort_key = w.template take<uint32_t>(size_t(n));
+  const int64_t chunks = cdiv(n, kNumChunk);
+  auto* slot = w.template take<int64_t>(size_t(n));
+  auto* place = w.template take<uint32_t>(size_t(n));
   auto* counts = w.template take<uint32_t>(size_t(max_vox));
   auto* start = w.template take<uint32_t>(size_t(max_vox));
-  auto* flags = w.template take<uint32_t>(64);
-  auto* tkeys = w.template take<uint64_t>(size_t(cap));
-  auto* tvals = w.template take<int32_t>(size_t(cap));
-  void* sws = w.template take<char>(sort_rows_ws_bytes(n));
-  void* cws = w.template take<char>(scan_workspace_bytes(scan_len));
+  auto* meta = w.template take<uint32_t>(kMetaWords + 2 * size_t(chunks));
+  auto* slots = w.template take<P2VSlot>(size_t(cap));
+  void* sws = w.template take<char>(sort_rows_ws_bytes(n));  // (at least 8 bytes a point)
   if (out) {
-    out->keys = reinterpret_cast<int64_t*>(keys);
-    out->first = reinterpret_cast<uint32_t*>(first);
-    out->rank = reinterpret_cast<uint32_t*>(rank);
-    out->sort_key = reinterpret_cast<uint32_t*>(sort_key);
-    out->counts = reinterpret_cast<uint32_t*>(counts);
-    out->start = reinterpret_cast<uint32_t*>(start);
-    out->n_unique = reinterpret_cast<uint32_t*>(flags);
-    out->overflow = reinterpret_cast<int*>(reinterpret_cast<uint32_t*>(flags) + 16);
-    out->tkeys = reinterpret_cast<uint64_t*>(tkeys);
-    out->tvals = reinterpret_cast<int32_t*>(tvals);
+    out->slot = slot;
+    out->place = place;
+    out->counts = counts;
+    out->start = start;
+    out->meta = meta;
+    out->state = reinterpret_cast<uint64_t*>(meta + kMetaWords);
+    out->slots = slots;
     out->sort_ws = sws;
-    out->scan_ws = cws;
     out->cap = cap;
+    out->chunks = chunks;
   }
 }
 
@@ -191,7 +332,7 @@ static void p2v_layout(W& w, int64_t n, int64_t max_vox, P2VWs* out) {
 static size_t p2v_ws_bytes(int64_t n, int64_t max_vox) {
   WsCursor c(nullptr, ~size_t(0));
   p2v_layout(c, n, max_vox, nullptr);
-  return c.off;
+  return c.off + 16;  // (the parts start at the workspace's first 16-byte boundary)
 }
 
 template <typename F>
@@ -200,54 +341,54 @@ static int p2v_run(const F* pc, int64_t n, int64_t cols, const P2VGeom& g, int n
                    int32_t* indices, int32_t* npv, int64_t* pc_voxel_id, int64_t* n_voxels,
                    const P2VWs& w, hipStream_t s) {
   const unsigned blocks = unsigned(cdiv(n, 256));
-  Table64 t{w.tkeys, w.tvals, w.cap - 1, w.overflow};
-  SP_HIP(hipMemsetAsync(w.n_unique, 0, 256, s));
-  SP_HIP(hipMemsetAsync(w.counts, 0, size_t(max_vox) * 4, s));
-  int rc = launch_fill_u64(w.tkeys, int64_t(w.cap), kEmpty64, s);
+  const P2VTable t{w.slots, w.cap - 1, w.meta + kMetaOverflow};
+  PinnedCounts counts;
+  int rc = counts.take();
   if (rc) return rc;
-  rc = launch_fill_i32(w.tvals, int64_t(w.cap), 0x7fffffff, s);
-  if (rc) return rc;
-  if (clear) {
-    rc = launch_fill<float>(voxels, max_vox * maxpts * nfeat, 0.f, s);
+  const int64_t n_vox = clear ? max_vox * maxpts * nfeat : 0;
+  const int64_t fb = cdiv(int64_t(w.cap) + n_vox / 4, 256);
+  p2v_clear<<<unsigned(fb < 4096 ? fb : 4096), 256, 0, s>>>(
+      reinterpret_cast<uint4*>(w.slots), int64_t(w.cap), w.meta, kMetaWords + 2 * w.chunks, voxels, n_vox);
+  SP_LAUNCHED();
+  p2v_insert<F><<<blocks, 256, 0, s>>>(pc, n, cols, g, t, p2v_rank_max(n, maxpts), w.meta, w.slot, w.place);
+  SP_LAUNCHED();
+  p2v_number<<<unsigned(w.chunks), kNumThreads, 0, s>>>(
+      w.slot, n, w.chunks, t, max_vox, maxpts, g, w.counts, w.start, npv, indices,
+      w.state, w.meta, counts.data());
+  SP_LAUNCHED();
+  SP_HIP(hipStreamSynchronize(s));
+  const int64_t found = int64_t(counts.data()[0]);
+  const int64_t nv = found < max_vox ? found : max_vox;
+  if (counts.data()[2])
+    return set_error(SP_ERR_HASH_FULL, "point2voxel: voxel hash overflowed");
+  const bool lists = counts.data()[1] == 0;
+  uint32_t* list = lists ? static_cast<uint32_t*>(w.sort_ws) : nullptr;
+  p2v_place<<<blocks, 256, 0, s>>>(w.slot, n, w.slots, max_vox, w.start, w.place, pc_voxel_id,
+                                   list);
+  const uint32_t* vid = w.place;
+  SP_LAUNCHED();
+  if (lists) {
+    p2v_rank<F><<<blocks, 256, 0, s>>>(pc, n, cols, nfeat, vid, w.counts, w.start, list, max_vox,
+                                       maxpts, voxels);
+    SP_LAUNCHED();
+  } else {
+    // stable sort of the points by voxel id (vid <= max_vox)
+    int bits = 0;
+    while ((uint64_t(1) << bits) <= uint64_t(max_vox)) ++bits;
+    const uint32_t mask = bits >= 32 ? 0xFFFFFFFFu : ((1u << bits) - 1u);
+    uint32_t* perm = nullptr;
+    rc = sort_rows_by_words(vid, n, 1, bits, mask, &perm, w.sort_ws, s);
     if (rc) return rc;
-  }
-  p2v_insert<F><<<blocks, 256, 0, s>>>(pc, n, cols, g, t, w.keys);
-  SP_LAUNCHED();
-  p2v_first<<<blocks, 256, 0, s>>>(w.keys, n, t, w.first);
-  SP_LAUNCHED();
-  rc = exclusive_scan_u32(w.first, w.rank, n, w.n_unique, w.scan_ws, s);
-  if (rc) return rc;
-  p2v_set_ids<<<blocks, 256, 0, s>>>(w.keys, n, t, w.first, w.rank);
-  SP_LAUNCHED();
-  p2v_assign<<<blocks, 256, 0, s>>>(w.keys, n, t, max_vox, pc_voxel_id, w.sort_key, w.counts);
-  SP_LAUNCHED();
-  // stable sort of the points by voxel id (sort_key <= max_vox)
-  int bits = 0;
-  while ((uint64_t(1) << bits) <= uint64_t(max_vox)) ++bits;
-  const uint32_t mask = bits >= 32 ? 0xFFFFFFFFu : ((1u << bits) - 1u);
-  uint32_t* perm = nullptr;
-  rc = sort_rows_by_words(w.sort_key, n, 1, bits, mask, &perm, w.sort_ws, s);
-  if (rc) return rc;
-  rc = exclusive_scan_u32(w.counts, w.start, max_vox, nullptr, w.scan_ws, s);
-  if (rc) return rc;
-  p2v_scatter<F><<<blocks, 256, 0, s>>>(pc, cols, nfeat, perm, w.sort_key, w.start, n, max_vox,
-                                        maxpts, voxels);
-  SP_LAUNCHED();
-  const unsigned vblocks = unsigned(cdiv(max_vox, 256));
-  p2v_voxels<<<vblocks, 256, 0, s>>>(w.counts, w.start, perm, w.keys, w.n_unique, max_vox, maxpts,
-                                     g, npv, indices);
-  SP_LAUNCHED();
-  if (empty_mean) {
-    const unsigned eblocks = unsigned(cdiv(max_vox * nfeat, 256));
-    p2v_empty_mean<<<eblocks, 256, 0, s>>>(voxels, npv, w.n_unique, max_vox, maxpts, nfeat);
+    p2v_scatter<F><<<blocks, 256, 0, s>>>(pc, cols, nfeat, perm, vid, w.start, n, max_vox,
+                                          maxpts, voxels);
     SP_LAUNCHED();
   }
-  uint32_t h[2] = {0, 0};
-  SP_HIP(hipMemcpyAsync(&h[0], w.n_unique, 4, hipMemcpyDeviceToHost, s));
-  SP_HIP(hipMemcpyAsync(&h[1], w.overflow, 4, hipMemcpyDeviceToHost, s));
-  SP_HIP(hipStreamSynchronize(s));
-  if (h[1]) return set_error(SP_ERR_HASH_FULL, "point2voxel: voxel hash overflowed");
-  *n_voxels = int64_t(h[0]) < max_vox ? int64_t(h[0]) : max_vox;
+  if (empty_mean && nv > 0) {
+    const unsigned eblocks = unsigned(cdiv(nv * nfeat, 256));
+    p2v_empty_mean<<<eblocks, 256, 0, s>>>(voxels, npv, nv, maxpts, nfeat);
+    SP_LAUNCHED();
+  }
+  *n_voxels = nv;
   return SP_OK;
 }
 
@@ -298,7 +439,8 @@ int sp_point2voxel(const void* points, int32_t dtype, int64_t n_points, int64_t 
   const size_t need = p2v_ws_bytes(n_points, max_voxels);
   if (!ws || ws_bytes < need)
     return set_error(SP_ERR_WORKSPACE, "point2voxel: workspace %zu < %zu", ws_bytes, need);
-  WsCursor c(ws, ws_bytes);
+  WsCursor c(reinterpret_cast<void*>((reinterpret_cast<uintptr_t>(ws) + 15) & ~uintptr_t(15)),
+             need - 16);
   P2VWs w;
   p2v_layout(c, n_points, max_voxels, &w);
   if (dtype == SP_F32)

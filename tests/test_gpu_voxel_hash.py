@@ -102,6 +102,28 @@ def test_point_to_voxel_matches_oracle(ci):
     _eq(res, _orc(ctor, pts), f"case {ci}")
 
 
+@pytest.mark.parametrize("n", [1, 1023, 1024, 1025, 140_001])
+@pytest.mark.parametrize("most,max_pts", [(1, 3), (8, 8), (9, 4), (119, 60), (120, 60), (256, 20),
+                                          (257, 20), (2000, 2)])
+def test_point_to_voxel_list_sizes(n, most, max_pts):
+    """Voxels of one point up to the most whose points are ranked by their
+    lists (256; 119 of 140001 with 60 kept), one past it and far past it
+    (sorted), with and without
+    truncation, around the chunk of the numbering scan (1024 points) and over
+    more chunks than one look-back step; half the voxels past the cap."""
+    g = torch.Generator().manual_seed(n + most)
+    vox = torch.arange(n) // most  # `most` points in each of them
+    pts = torch.rand(n, 4, generator=g) * 0.5 + 0.25
+    for d in range(3):
+        pts[:, d] += (vox // 60 ** d % 60).float()
+    pts = pts[torch.randperm(n, generator=g)]
+    ctor = dict(vsize_xyz=[1.0] * 3, coors_range_xyz=[0.0] * 3 + [60.0] * 3,
+                num_point_features=4, max_num_voxels=max(1, n // most // 2),
+                max_num_points_per_voxel=max_pts)
+    _, res = _p2v(ctor, pts)
+    _eq(res, _orc(ctor, pts), f"n {n} most {most}")
+
+
 def test_point_to_voxel_empty_mean():
     """empty_mean fills empty slots with the voxel's mean (the sum over all
     slots, in slot order, over the clamped count: one rounding order of the
