@@ -377,8 +377,8 @@ int sp_conv_wgrad(const void* x, int64_t n_in, const void* g, int64_t n_out, int
                   void* dw, void* ws, size_t ws_bytes, void* stream);
 
 /* Eval-mode BatchNorm over rows [rows, C] (f16/bf16/f32):
- * out = (x - mean) * (weight / sqrt(var + eps)) + bias in fp32, rounded, and max(out, 0) with
- * relu (a NaN stays).  mean, var, weight and bias [C] in param_dtype (the rows' type or fp32);
+ * out = fma(weight * (x - mean), rsqrt(var + eps), bias) in fp32, rounded, and max(out, 0) with
+ * relu (a NaN stays): bit for bit what torch's modules give.  mean, var, weight and bias [C] in param_dtype (the rows' type or fp32);
  * weight and bias nullable (1 and 0).  The reference runs torch's modules here. */
 int sp_batchnorm_eval(const void* x, int32_t dtype, int64_t rows, int64_t C, const void* mean,
                       const void* var, const void* weight, const void* bias, int32_t param_dtype,

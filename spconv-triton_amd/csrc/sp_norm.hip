@@ -1,6 +1,9 @@
 // Eval-mode BatchNorm over feature rows, with or without a ReLU after it, in one
-// pass: y = (x - mean) * (weight / sqrt(var + eps)) + bias, rounded to the rows'
-// type, then max(y, 0) (a NaN stays).
+// pass: y = fma(weight * (x - mean), rsqrt(var + eps), bias) in fp32, rounded to
+// the rows' type, then max(y, 0) (a NaN stays).  The steps and their order are
+// those that torch's modules show (compared bit for bit in every type): weight *
+// rsqrt taken first, as one scale a channel, flips last bits of 16-bit rows,
+// which the layers after it carry on.
 //
 // Bound by memory: the rows are read and written once.  A thread holds one
 // 16-byte piece of the channels for kNormRows rows, all loaded at once, the
@@ -21,8 +24,13 @@ __device__ __forceinline__ float norm_param(const void* p, int c, float none) {
 }
 
 template <typename T>
-__device__ __forceinline__ T norm_one(float x, float mean, float scale, float shift, bool relu) {
-  const T y = T((x - mean) * scale + shift);
+__device__ __forceinline__ T norm_one(float x, float mean, float weight, float inv, float bias,
+                                      bool relu) {
+  float r = __builtin_fmaf(weight * (x - mean), inv, bias);
+  // rounded to fp32 first: without this, the fp16 instances take the fused
+  // multiply-add that rounds once, to fp16 (about 1 value in 16 000 differs)
+  asm("" : "+v"(r));
+  const T y = T(r);
   return relu && y < T(0) ? T(0) : y;
 }
 
@@ -36,7 +44,7 @@ __global__ __launch_bounds__(kNormThreads) void batchnorm_rows(
     const void* __restrict__ var, const void* __restrict__ weight, const void* __restrict__ bias,
     float eps, int relu, T* __restrict__ out) {
   using vec = __attribute__((ext_vector_type(V))) T;
-  extern __shared__ float s_par[];  // mean, scale, shift: C each
+  extern __shared__ float s_par[];  // mean, weight, 1 / deviation, bias: C each
   const int per = kNormThreads / pieces;  // rows side by side
   const int r0 = int(threadIdx.x) / pieces, c0 = (int(threadIdx.x) - r0 * pieces) * V;
   const int64_t base = int64_t(blockIdx.x) * (per * kNormRows) + r0;
@@ -49,17 +57,19 @@ __global__ __launch_bounds__(kNormThreads) void batchnorm_rows(
   }
   for (int c = int(threadIdx.x); c < C; c += kNormThreads) {
     s_par[c] = norm_param<P>(mean, c, 0.f);
-    s_par[C + c] = norm_param<P>(weight, c, 1.f) / sqrtf(norm_param<P>(var, c, 1.f) + eps);
-    s_par[2 * C + c] = norm_param<P>(bias, c, 0.f);
+    s_par[C + c] = norm_param<P>(weight, c, 1.f);
+    s_par[2 * C + c] = rsqrtf(norm_param<P>(var, c, 1.f) + eps);
+    s_par[3 * C + c] = norm_param<P>(bias, c, 0.f);
   }
   __syncthreads();
   if (idle) return;
-  float m[V], sc[V], sh[V];
+  float m[V], w[V], inv[V], b[V];
 #pragma unroll
   for (int i = 0; i < V; ++i) {
     m[i] = s_par[c0 + i];
-    sc[i] = s_par[C + c0 + i];
-    sh[i] = s_par[2 * C + c0 + i];
+    w[i] = s_par[C + c0 + i];
+    inv[i] = s_par[2 * C + c0 + i];
+    b[i] = s_par[3 * C + c0 + i];
   }
 #pragma unroll
   for (int j = 0; j < kNormRows; ++j) {
@@ -67,7 +77,8 @@ __global__ __launch_bounds__(kNormThreads) void batchnorm_rows(
     if (r >= rows) continue;
     vec y;
 #pragma unroll
-    for (int i = 0; i < V; ++i) y[i] = norm_one<T>(float(v[j][i]), m[i], sc[i], sh[i], relu != 0);
+    for (int i = 0; i < V; ++i)
+      y[i] = norm_one<T>(float(v[j][i]), m[i], w[i], inv[i], b[i], relu != 0);
     *reinterpret_cast<vec*>(out + r * C + c0) = y;
   }
 }
@@ -81,10 +92,9 @@ __global__ __launch_bounds__(kNormThreads) void batchnorm_values(
   const int64_t step = int64_t(gridDim.x) * kNormThreads;
   for (int64_t i = int64_t(blockIdx.x) * kNormThreads + threadIdx.x; i < n; i += step) {
     const int c = int(i % C);
-    const float scale =
-        norm_param<P>(weight, c, 1.f) / sqrtf(norm_param<P>(var, c, 1.f) + eps);
-    out[i] = norm_one<T>(float(x[i]), norm_param<P>(mean, c, 0.f), scale,
-                         norm_param<P>(bias, c, 0.f), relu != 0);
+    out[i] = norm_one<T>(float(x[i]), norm_param<P>(mean, c, 0.f), norm_param<P>(weight, c, 1.f),
+                         rsqrtf(norm_param<P>(var, c, 1.f) + eps), norm_param<P>(bias, c, 0.f),
+                         relu != 0);
   }
 }
 
@@ -101,7 +111,7 @@ static int run_batchnorm(const void* x, int64_t rows, int C, const void* mean, c
     const int pieces = C / V;
     const int64_t blocks = cdiv(rows, int64_t(kNormThreads / pieces) * kNormRows);
     SP_CHECK_ARG(blocks <= kMaxGridX, "batchnorm: too many rows");
-    batchnorm_rows<T, P, V><<<unsigned(blocks), kNormThreads, 3 * C * sizeof(float), s>>>(
+    batchnorm_rows<T, P, V><<<unsigned(blocks), kNormThreads, 4 * C * sizeof(float), s>>>(
         xt, rows, C, pieces, mean, var, weight, bias, eps, relu, ot);
   } else {
     const int64_t blocks = cdiv(rows * C, kNormThreads);

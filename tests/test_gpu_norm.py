@@ -77,6 +77,29 @@ def test_batchnorm_special_values():
     assert torch.equal(torch.isinf(y), torch.isinf(t))
 
 
+@pytest.mark.parametrize("rows,C,dtype,pdtype,affine", [
+    (1, 16, F16, F16, True), (20000, 64, F16, F16, True), (3001, 33, F16, F32, True),
+    (3000, 2056, F16, F16, True), (5000, 128, F16, F16, False), (9000, 48, BF16, BF16, True),
+    (2000, 5, BF16, F32, False), (9000, 64, F32, F32, True), (700, 300, F32, F32, False),
+    (129, 1030, F32, F32, True)])
+def test_batchnorm_eval_is_torch_bit_for_bit(rows, C, dtype, pdtype, affine):
+    """The steps and their order are the module's, so a network's values do not depend on
+    whether its BatchNorm and ReLU are fused."""
+    import spconv_triton.pytorch as spconv
+
+    torch.manual_seed(rows + C)
+    x = (torch.randn(rows, C, device=DEV) * 2).to(dtype)
+    bn = _bn(C, pdtype, affine, seed=C)
+    x[0] = bn.running_mean.to(dtype)
+    bits = torch.int32 if dtype is F32 else torch.int16
+    with torch.no_grad():
+        t = bn(x)
+        for net, ref in ((spconv.SparseSequential(bn), t),
+                         (spconv.SparseSequential(bn, nn.ReLU()), torch.relu(t))):
+            y = net(_tensor(x)).features
+            assert torch.equal(y.view(bits), ref.view(bits))
+
+
 class _MyBN(nn.BatchNorm1d):
     def forward(self, x):
         return super().forward(x) + 1
