@@ -31,13 +31,15 @@ def _plain(mod: nn.Module) -> bool:
 def passes_unobserved() -> bool:
     """No gradient, global hook, mode, trace or transform could see a module or
     tensor operation of this pass."""
+    if torch.compiler.is_compiling():  # (first: Dynamo cannot trace the questions below)
+        return False
     return not (torch.is_grad_enabled() or _module._global_forward_hooks
                 or _module._global_forward_pre_hooks or _module._global_backward_hooks
                 or _module._global_backward_pre_hooks
                 or torch._C._len_torch_dispatch_stack() or torch._C._len_torch_function_stack()
                 or torch._C._functorch.peek_interpreter_stack() is not None
                 or torch.autograd.forward_ad._current_level >= 0
-                or torch.compiler.is_compiling() or torch.jit.is_tracing()
+                or torch.jit.is_tracing()
                 or nn.Module.__call__ is not _CALL)
 
 
