@@ -2,9 +2,9 @@
 
 ``SparseSequential`` hands the plain ``nn.BatchNorm1d`` (and the ``nn.ReLU``
 after it) of an inference pass here (``sp_batchnorm_eval``).  ``fusable_bn`` and
-``fusable_relu`` accept exactly the modules whose call does nothing else: no
-subclass, hook, replaced ``forward``, training mode, gradient, tracing or
-transform; everything else runs the modules themselves.
+``fusable_relu`` accept only modules whose call does nothing else: no
+subclass (of module or tensors), hook, replaced ``forward``, training mode,
+gradient, tracing or transform; everything else runs the modules themselves.
 """
 
 from __future__ import annotations
@@ -19,6 +19,7 @@ _BN_FORWARD = nn.BatchNorm1d.forward
 _RELU_FORWARD = nn.ReLU.forward
 _CALL = nn.Module.__call__
 _FLOATS = (torch.float16, torch.bfloat16, torch.float32)
+_TENSORS = (torch.Tensor, nn.Parameter)
 
 
 def _plain(mod: nn.Module) -> bool:
@@ -47,36 +48,50 @@ def fusable_relu(mod: nn.Module) -> bool:
     return type(mod) is nn.ReLU and nn.ReLU.forward is _RELU_FORWARD and _plain(mod)
 
 
+def _statistics(mod: nn.BatchNorm1d):
+    """What the module's forward reads, as it reads it (also where an instance attribute
+    has taken a parameter's place)."""
+    return mod.running_mean, mod.running_var, mod.weight, mod.bias
+
+
+def _plain_tensor(t) -> bool:
+    """The values of ``t`` are its memory's: no subclass, whose operations are its own and whose
+    memory may be none, no lazy negation or zeros."""
+    return type(t) in _TENSORS and not t.is_neg() and not t._is_zerotensor()
+
+
 def fusable_bn(mod: nn.Module, x: torch.Tensor) -> bool:
     """``mod`` is a plain eval BatchNorm1d over the rows of ``x`` that torch would
     compute from its running statistics, in types this kernel has."""
     if not (type(mod) is nn.BatchNorm1d and nn.BatchNorm1d.forward is _BN_FORWARD
             and not mod.training and _plain(mod)):
         return False
-    params = mod._parameters
-    weight, bias = params.get("weight"), params.get("bias")
-    mean, var = mod._buffers.get("running_mean"), mod._buffers.get("running_var")
     if not (type(x) is torch.Tensor and x.is_cuda and x.dim() == 2 and x.is_contiguous()
-            and x.dtype in _FLOATS and 0 < x.shape[1] < 65536
-            and mean is not None and var is not None):
+            and x.dtype in _FLOATS and 0 < x.shape[1] < 65536 and _plain_tensor(x)):
+        return False
+    return _fusable_statistics(_statistics(mod), x.dtype, x.device, x.shape[1])
+
+
+def _fusable_statistics(stats, dtype, dev, width: int) -> bool:
+    mean, var, weight, bias = stats
+    if mean is None or var is None:
         return False
     want = mean.dtype
-    if want is not x.dtype and want is not torch.float32:
+    if want is not dtype and want is not torch.float32:
         return False
-    width, dev = x.shape[1], x.device
-    for t in (mean, var, weight, bias):
-        if t is not None and not (t.dtype is want and t.device == dev and t.dim() == 1
-                                  and t.shape[0] == width and t.is_contiguous()):
+    for t in stats:
+        if t is not None and not (_plain_tensor(t) and t.dtype is want and t.device == dev
+                                  and t.dim() == 1 and t.shape[0] == width
+                                  and t.is_contiguous()):
             return False
     return True
 
 
 def batchnorm_eval(mod: nn.Module, x: torch.Tensor, relu: bool) -> torch.Tensor:
     out = torch.empty_like(x)
-    mean, var = mod._buffers["running_mean"], mod._buffers["running_var"]
+    mean, var, weight, bias = _statistics(mod)
     _lib.check(_lib.lib().sp_batchnorm_eval(
         _lib.ptr(x), _lib.dtype_code(x.dtype), x.shape[0], x.shape[1], _lib.ptr(mean),
-        _lib.ptr(var), _lib.ptr(mod._parameters.get("weight")),
-        _lib.ptr(mod._parameters.get("bias")), _lib.dtype_code(mean.dtype), float(mod.eps),
-        int(relu), _lib.ptr(out), _lib.stream_of(x.device)), "sp_batchnorm_eval")
+        _lib.ptr(var), _lib.ptr(weight), _lib.ptr(bias), _lib.dtype_code(mean.dtype),
+        float(mod.eps), int(relu), _lib.ptr(out), _lib.stream_of(x.device)), "sp_batchnorm_eval")
     return out

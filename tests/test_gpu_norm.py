@@ -139,3 +139,39 @@ def test_observed_modules_run_themselves(monkeypatch):
         assert len(calls) == n
     y = net(_tensor(x.clone().requires_grad_(True))).features
     assert y.requires_grad and len(calls) == n
+
+
+class _Doubled(torch.Tensor):
+    """A tensor without memory of its own whose value is twice the one it holds."""
+
+    @staticmethod
+    def __new__(cls, inner):
+        return torch.Tensor._make_wrapper_subclass(cls, inner.shape, dtype=inner.dtype,
+                                                   device=inner.device)
+
+    def __init__(self, inner):
+        self.inner = inner
+
+    @classmethod
+    def __torch_dispatch__(cls, func, types, args=(), kwargs=None):
+        args = [a.inner * 2 if isinstance(a, cls) else a for a in args]
+        return func(*args, **(kwargs or {}))
+
+
+def test_other_parameters_than_plain_tensors():
+    """A wrapper-subclass weight runs torch's module; an attribute in a parameter's place is the
+    weight of the fused launch too."""
+    import spconv_triton.pytorch as spconv
+
+    x = torch.randn(100, 16, device=DEV)
+    bn = _bn(16, F32)
+    weight = bn.weight.detach().clone()
+    net = spconv.SparseSequential(bn, nn.ReLU())
+    with torch.no_grad():
+        bn.weight.mul_(2)
+        want = torch.relu(bn(x))
+        bn._parameters["weight"] = _Doubled(weight)
+        assert torch.equal(net(_tensor(x)).features, want)
+        del bn.weight
+        bn.weight = weight * 2
+        assert torch.equal(net(_tensor(x)).features, want)
