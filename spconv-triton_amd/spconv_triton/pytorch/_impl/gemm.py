@@ -137,25 +137,34 @@ def packed_weight(filters: torch.Tensor, bias: torch.Tensor | None, dtype,
 #: the two kernels.
 USE_GATHER_PLAN = "auto"
 PLAN_MIN_WORK = 100_000 * 64
-#: Outputs of at most NARROW_COLS columns run the narrow kernel when no plan is
-#: used, which multiplies 32 columns where the planned kernels multiply 64 (and
-#: skips fp32 blocks without a pair).  With fp32 operands, or 16-bit rows of at
-#: most NARROW_SHORT_ROW elements (one K-step an offset), it beats them at every
-#: size measured, before the plan's own build (us, planned -> narrow): 240k urban
-#: rows fp32 32 -> 32 146 -> 80, fp16 16 -> 32 23.2 -> 19.3; 200k surface rows
-#: fp32 64 -> 32 373 -> 237, fp16 3 -> 32 46 -> 39.  Longer 16-bit rows keep the
-#: rule above (200k surface rows fp16 64 -> 32 45 -> 55; 240k urban 42 -> 40).
+#: Outputs of at most NARROW_COLS columns run the narrow kernel when neither a plan
+#: nor a row order is used; it multiplies 32 columns where the planned kernels
+#: multiply 64 (and skips fp32 blocks without a pair).  With fp32 operands, or 16-bit
+#: rows of at most NARROW_SHORT_ROW elements (one K-step an offset), it beats them in
+#: natural order at every size measured, before the plan's own build (us, planned ->
+#: narrow): 240k urban rows fp32 32 -> 32 146 -> 80, fp16 16 -> 32 23.2 -> 19.3; 200k
+#: surface rows fp32 64 -> 32 373 -> 237, fp16 3 -> 32 46 -> 39; a random permutation of
+#: their rows 441 (in key order) -> 239 and 51 -> 39.  Longer 16-bit rows keep the rule
+#: above (200k surface rows fp16 64 -> 32 45 -> 55; 240k urban 42 -> 40), and so does a
+#: table in mask order, where the kernel without a plan is the 64-column one (planned ->
+#: unplanned: 50k LiDAR rows fp32 256 -> 32 178 -> 411, 240k urban rows fp32 64 -> 32
+#: 105 -> 205, fp16 16 -> 32 29 -> 38).
 NARROW_COLS = 32
 NARROW_SHORT_ROW = 16
 
 
-def _use_plan(M: int, C: int, K: int, cols: int, row: int, dtype) -> bool:
-    """cols: columns of the output; row, dtype: elements of a source row and their type."""
-    if USE_GATHER_PLAN != "auto":
-        return bool(USE_GATHER_PLAN)
-    if cols <= NARROW_COLS and (dtype == torch.float32 or row <= NARROW_SHORT_ROW):
-        return False
-    return M * max(C, K) >= PLAN_MIN_WORK
+def _use_plan(M: int, C: int, K: int) -> bool:
+    if USE_GATHER_PLAN == "auto":
+        return M * max(C, K) >= PLAN_MIN_WORK
+    return bool(USE_GATHER_PLAN)
+
+
+def _narrow(cols: int, row: int, dtype, out_dtype) -> bool:
+    """In natural order the narrow kernel is taken instead of a plan.  cols: columns of the
+    output; row, dtype: elements of a source row and their type."""
+    return (USE_GATHER_PLAN == "auto" and cols <= NARROW_COLS
+            and out_dtype in (dtype, torch.float32)  # (the types the kernel writes)
+            and (dtype == torch.float32 or row <= NARROW_SHORT_ROW))
 
 
 def gather_plan(pairs: torch.Tensor, n_src: int, words: torch.Tensor | None = None):
@@ -508,9 +517,11 @@ def _gemm(a: torch.Tensor, filters: torch.Tensor, bias, transpose: bool, pairs: 
     kv = pairs.shape[0]
     packed = packed_weight(filters, bias, "bf16x3" if split else a.dtype, transpose)
     L = _lib.lib()
-    use_plan = _use_plan(M, C, K, C if transpose else K, a.shape[1], a.dtype)
+    use_plan = _use_plan(M, C, K)
     variant = row_order_variant(pairs, a.shape[0], K * C, use_plan,
                                 fp32=a.dtype == torch.float32 and not split)
+    if variant is None and _narrow(C if transpose else K, a.shape[1], a.dtype, out.dtype):
+        use_plan = False
     if split:  # the GEMM's reduction dimension is tripled
         K, C = (3 * K, C) if transpose else (K, 3 * C)
     if variant is None:

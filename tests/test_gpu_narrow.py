@@ -60,3 +60,42 @@ def test_narrow_large_window_matches_fp64():
         mag[o] += xi.abs() @ w[:, k].double().abs().T
     # at most 150 * 24 fp32 sums of exact-to-rounding products
     assert ((y.double() - ref).abs() <= 2.0 ** -24 * 200 * mag + 1e-30).all()
+
+
+@pytest.mark.parametrize("C,K,dtype", [(64, 32, torch.float32), (16, 32, torch.float16),
+                                       (4, 16, torch.bfloat16)])
+def test_a_table_in_mask_order_keeps_its_plan(C, K, dtype, monkeypatch):
+    """A narrow layer on a table whose rows are taken in mask order runs the planned kernel: the
+    narrow one takes natural rows only.  The result is that of the narrow kernel."""
+    from spconv_triton.pytorch._impl import gemm
+
+    rng = np.random.default_rng(C)
+    kv, M = 27, 1500
+    t = rng.integers(0, M, size=(kv, M)).astype(np.int32)
+    t[rng.random((kv, M)) >= 0.1] = -1
+    x = torch.randn(M, C, device=DEV).to(dtype)
+    w = torch.randn(K, kv, C, device=DEV).to(dtype)
+    monkeypatch.setattr(gemm, "PLAN_MIN_WORK", M * K)
+    plain = torch.from_numpy(t).to(DEV)
+    monkeypatch.setattr(gemm, "ROW_ORDER", "natural")
+    want = gemm.conv_forward(x, w, plain, M)
+    assert not hasattr(plain, "_spconv_triton_plan")  # the narrow kernel
+    ordered = torch.from_numpy(t).to(DEV)
+    monkeypatch.setattr(gemm, "ROW_ORDER", "mask")
+    got = gemm.conv_forward(x, w, ordered, M)
+    assert ordered._spconv_triton_order[1][2] is not None
+    assert torch.equal(got, want)
+
+
+def test_output_types_the_narrow_kernel_does_not_write_are_planned(monkeypatch):
+    from spconv_triton.pytorch._impl import gemm
+
+    monkeypatch.setattr(gemm, "ROW_ORDER", "natural")
+    monkeypatch.setattr(gemm, "PLAN_MIN_WORK", 1)
+    tab = torch.arange(300, dtype=torch.int32, device=DEV).view(1, -1)
+    x = torch.randn(300, 8, device=DEV).half()
+    w = torch.randn(8, 1, 8, device=DEV).half()
+    y = gemm.conv_forward(x, w, tab, 300, out_dtype=torch.bfloat16)
+    assert hasattr(tab, "_spconv_triton_plan")
+    ref = gemm.conv_forward(x, w, tab, 300, out_dtype=torch.float32)
+    assert torch.equal(y, ref.bfloat16())
