@@ -90,12 +90,15 @@ class SparseSequential(SparseModule):
                 x = module(x)
             elif isinstance(x, sct):
                 if x.indices.shape[0] != 0:
-                    if (type(module) is nn.BatchNorm1d and _norm.passes_unobserved()
-                            and _norm.fusable_bn(module, x.features)):
+                    stats = None
+                    if type(module) is nn.BatchNorm1d and _norm.passes_unobserved():
+                        stats = _norm.fusable_bn(module, x.features)
+                    if stats is not None:
                         # an inference pass's plain BatchNorm1d, with the plain ReLU after it
                         relu = i < len(mods) and _norm.fusable_relu(mods[i])
                         i += relu
-                        x = x.replace_feature(_norm.batchnorm_eval(module, x.features, relu))
+                        x = x.replace_feature(
+                            _norm.batchnorm_eval(module, x.features, relu, stats))
                         continue
                     x = x.replace_feature(module(x.features))
             else:

@@ -159,8 +159,7 @@ class _Doubled(torch.Tensor):
 
 
 def test_other_parameters_than_plain_tensors():
-    """A wrapper-subclass weight runs torch's module; an attribute in a parameter's place is the
-    weight of the fused launch too."""
+    """A wrapper-subclass weight, or an attribute in the parameter's place, counts."""
     import spconv_triton.pytorch as spconv
 
     x = torch.randn(100, 16, device=DEV)
