@@ -889,16 +889,40 @@ __global__ __launch_bounds__(256, 2) void gather_gemm_direct(
 // ---------------------------------------------------------------------------
 // direct_tile's 64 x 64 waves would spend half their MFMAs, weight loads and
 // accumulators on columns that do not exist; 64 rows x 32 columns take 106
-// registers, so four workgroups fit on a CU instead of two and hide the gathers
-// for each other.  Same items and summation order: results are bit-identical.
-// Bound by the gathers' latency: two steps in flight and four workgroups a CU
-// measured as well as three or four steps and three.  Measured without a gather
+// registers and, for a 3x3x3 window, at most 37 KB of LDS (narrow_lds), so four
+// workgroups fit on a CU instead of two and hide the gathers for each other.
+// Same items and summation order: results are bit-identical.
+// Bound by the gathers' latency.  (With direct_lds's bytes, 41 KB and 70 KB of
+// fp32 output, three and two fitted: 240k urban rows fp32 32 -> 32 80.5 -> 73.5
+// us, 400k rows of a 1024^3 surface fp32 64 -> 32 356 -> 322, fp16 16 -> 32 35.2
+// -> 29.5.)  Measured with those, and without a gather
 // plan (us, direct -> narrow, and the staged kernel without its plan's build,
 // ~25 us a table; fp16 unless said): LiDAR encoder 80k rows 4 -> 16 30.7 -> 14.4
 // (22.7), 193k rows 16 -> 32 38.2 -> 15.9 (22.0), 32 -> 32 40.2 -> 27.0 (27.7);
 // 80k rows fp32 48 -> 20 137 -> 70 (130); 2 000 rows fp32 16 -> 16 24.7 -> 14.  Two
 // such blocks for 64 columns gather every row twice: slower than direct_tile
 // (metric layer 80 -> 85, urban 64 -> 64 54 -> 62).
+
+// Dynamic LDS of the narrow kernel, per wave: an entry for each of a group's items
+// and one padding item; direct_tile's A slots only in the instances that use them
+// (slot); the epilogue's 32 x 32 tile overlaps the tables.
+__host__ __device__ constexpr DirectLds narrow_lds(int G, uint32_t out_size, bool slot) {
+  const uint32_t E = uint32_t(G) + 1u, epilogue = 4u * 32u * (32u * out_size + 16u);
+  DirectLds l{};
+  l.kb_off = 0;
+  l.src_off = (16u * E + 255u) / 256u * 256u;
+  l.a_off = l.src_off + E * 1024u;
+  l.total = l.a_off + (slot ? 4u * 2048u : 0u);
+  if (l.total < l.src_off + epilogue) l.total = l.src_off + epilogue;
+  return l;
+}
+static_assert(4u * narrow_lds(27, 4, false).total <= 160u * 1024u &&
+                  4u * narrow_lds(27, 2, true).total <= 160u * 1024u,
+              "four workgroups of a 3x3x3 window fit in a CU's LDS");
+// (in which the A slots are used: whole chunks of 16-bit rows)
+__host__ __device__ constexpr bool narrow_slot(int rowb, int ks, size_t elem) {
+  return rowb == 16 && ks == 2 && elem == 2;
+}
 
 // ROWB: what a row is a whole number of: 16-byte pieces, 8-byte halves of them, or
 // elements (0).  KS: K-steps of an item; 1 for rows of at most 2 V elements,
@@ -914,7 +938,7 @@ __global__ __launch_bounds__(256, ROWB == 0 && KS == 2 ? 3 : 4) void gather_gemm
   constexpr int kChunk = kChunkBytes / int(ES);
   constexpr int DEPTH = 2;  // steps of A rows and weights in flight
   // row-contiguous loads through an LDS slot, as in direct_tile (whole chunks only)
-  constexpr bool SLOT = ROWB == 16 && sizeof(T) == 2 && KS == 2;
+  constexpr bool SLOT = narrow_slot(ROWB, KS, sizeof(T));
   // fp32 MFMAs take 8 x as long a product: those of a 32-row block without a pair are skipped
   constexpr bool SKIP = sizeof(T) == 4;
   extern __shared__ __align__(16) unsigned char smem[];
@@ -932,8 +956,8 @@ __global__ __launch_bounds__(256, ROWB == 0 && KS == 2 ? 3 : 4) void gather_gemm
   const __amdgpu_buffer_rsrc_t rp = make_rsrc(pairs, nb.pairs_bytes);
 
   const int G = kv < kGroupOffsets ? kv : kGroupOffsets;
-  const int E = G + kPad;
-  const DirectLds L = direct_lds(E, uint32_t(sizeof(OutT)));
+  const int E = G + 1;
+  const DirectLds L = narrow_lds(G, uint32_t(sizeof(OutT)), SLOT);
   uint32_t* s_kb = reinterpret_cast<uint32_t*>(smem + L.kb_off) + wave * E;
   uint32_t* s_src = reinterpret_cast<uint32_t*>(smem + L.src_off) + wave * E * 64;
   unsigned char* aslot = smem + L.a_off + uint32_t(wave) * 2048u;

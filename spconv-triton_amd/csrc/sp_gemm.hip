@@ -687,7 +687,6 @@ static int launch_narrow(hipStream_t s, const T* A, const T* bt, const int32_t* 
                          GemmBufs nb, const GemmCall& c) {
   constexpr int V = Mfma<T>::V;
   const int G = c.kv < kGroupOffsets ? c.kv : kGroupOffsets;
-  const uint32_t lds = direct_lds(G + kPad, uint32_t(sizeof(OutT))).total;
   using Kern = decltype(&gather_gemm_narrow<T, OutT, 16, 2>);
   constexpr Kern kerns[3][2] = {
       {gather_gemm_narrow<T, OutT, 16, 1>, gather_gemm_narrow<T, OutT, 16, 2>},
@@ -696,9 +695,11 @@ static int launch_narrow(hipStream_t s, const T* A, const T* bt, const int32_t* 
   const bool halves = int64_t(c.R) * int64_t(sizeof(T)) % 8 == 0 &&
                       reinterpret_cast<uintptr_t>(A) % 8 == 0;
   const int row = c.vec ? 0 : halves ? 1 : 2, ks = c.R <= 2 * V ? 0 : 1;
+  const bool slot = narrow_slot(row == 0 ? 16 : row == 1 ? 8 : 0, ks + 1, sizeof(T));
+  const uint32_t lds = narrow_lds(G, uint32_t(sizeof(OutT)), slot).total;
   static bool attr_set[3][2] = {};  // per kernel instance
   int rc = allow_lds(reinterpret_cast<const void*>(kerns[row][ks]),
-                     direct_lds(kGroupOffsets + kPad, uint32_t(sizeof(OutT))).total,
+                     narrow_lds(kGroupOffsets, uint32_t(sizeof(OutT)), slot).total,
                      attr_set[row][ks]);
   if (rc) return rc;
   kerns[row][ks]<<<dim3(unsigned(cdiv(c.M, kTileRows))), 256, lds, s>>>(
