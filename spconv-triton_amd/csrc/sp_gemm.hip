@@ -189,6 +189,8 @@ __device__ __forceinline__ typename Mfma<T>::frag load_frag_vec(const T* p) {
 // `per` of its pairs, `per` a whole number of stages and the same for all
 // offsets: all workgroups run about as long.  The fp32 partial of each share
 // is summed in ascending share by wgrad_reduce (deterministic, no atomics).
+// The pairs are known on the device only, so every wave works its share out
+// from the offsets' counts, by itself (block-wide scans took 3 us more a call).
 //
 // Pairs per share: the total over `target` shares, in whole stages.
 __device__ __forceinline__ int64_t wg_per(int64_t total, int target, int stage) {
@@ -196,18 +198,22 @@ __device__ __forceinline__ int64_t wg_per(int64_t total, int target, int stage) 
   return (stages > 0 ? stages : 1) * stage;
 }
 
-// Sum over the workgroup's NT threads, in a fixed order; red holds NT / 64.
-template <int NT>
-__device__ __forceinline__ int64_t wg_block_sum(int64_t v, int64_t* red) {
+__device__ __forceinline__ int64_t wave_sum(int64_t v) {
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) v += __shfl_xor(v, off, 64);
-  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
-  __syncthreads();
-  int64_t t = 0;
-#pragma unroll
-  for (int w = 0; w < NT / 64; ++w) t += red[w];
-  __syncthreads();
-  return t;
+  return v;
+}
+
+// Shares of an offset with cnt pairs.
+__device__ __forceinline__ int wg_count(int32_t cnt, int64_t per) {
+  const uint32_t p = per < 0x7fffffff ? uint32_t(per) : 0x7fffffffu;
+  return int((uint32_t(cnt) + p - 1u) / p);
+}
+
+__device__ __forceinline__ int64_t wg_total(const int32_t* __restrict__ counts, int kv, int lane) {
+  int64_t total = 0;
+  for (int k = lane; k < kv; k += 64) total += counts[k];
+  return wave_sum(total);
 }
 
 template <typename T, int BW>
@@ -223,14 +229,22 @@ struct WgShape {
   static_assert(2 * BW * kPitch * sizeof(T) <= 72 * 1024, "wgrad LDS");
 };
 
+// LDS holds two workgroups of the 128-wide shapes.  Without the bound they take up to
+// 266 registers a lane and one fits (fp32 256 -> 256, 75k surface rows 662 -> 491 us);
+// 16-bit element-wise rows on both sides, 256 + 64, spill too much under it.
+__host__ __device__ constexpr int wg_min_waves(int vec, int bw, size_t elem) {
+  return bw == 128 && (vec != 0 || elem == 4) ? 2 : 1;
+}
+
 // VEC bit 0: X rows are whole 16-byte vectors (C % V == 0, aligned base),
 // bit 1: the same for the G rows; otherwise that tensor is read element-wise.
 template <typename T, int VEC, int BW>
-__global__ __launch_bounds__(256) void wgrad_partial(
+__global__ __launch_bounds__(256, (wg_min_waves(VEC, BW, sizeof(T)))) void wgrad_partial(
     const T* __restrict__ X, int64_t n_in, const T* __restrict__ G, int64_t n_out, int C, int K,
     int kv, const int32_t* __restrict__ in_rows, const int32_t* __restrict__ out_rows,
     const int32_t* __restrict__ counts, int64_t stride, int target, int slots,
-    float* __restrict__ part, uint32_t x_bytes, uint32_t g_bytes, int cblocks, int nblocks) {
+    float* __restrict__ part, int32_t* __restrict__ first, uint32_t x_bytes, uint32_t g_bytes,
+    int cblocks, int nblocks) {
   using MF = Mfma<T>;
   using frag = typename MF::frag;
   using S = WgShape<T, BW>;
@@ -254,10 +268,6 @@ __global__ __launch_bounds__(256) void wgrad_partial(
     return COAL ? ((((p >> 3) ^ (((c >> 4) & 1) << 2)) << 3) | (p & 7)) : p;
   };
 
-  __shared__ int64_t s_red[4];
-  __shared__ uint32_t s_scan[5];
-  __shared__ int s_found[2];
-
   // share `slot` and (c, n) block of this workgroup: the cblocks * nblocks
   // blocks of one share gather the same pairs' rows (each input row for every
   // n block, each gradient row for every c block), so they run back to back on
@@ -268,31 +278,36 @@ __global__ __launch_bounds__(256) void wgrad_partial(
   const int slot = int((t / bpk) * 8 + blockIdx.x % 8);
   if (slot >= slots) return;  // padding of the last group of 8 shares
   const int blk = int(t % bpk);
-  int64_t total = 0;
-  for (int kk = threadIdx.x; kk < kv; kk += 256) total += counts[kk];
-  total = wg_block_sum<256>(total, s_red);
-  const int64_t per = wg_per(total, target, STAGE);
-  if (threadIdx.x == 0) s_found[0] = -1;
-  uint32_t before = 0;
-  for (int kb = 0; kb < kv; kb += 256) {  // the offset whose shares hold `slot`
-    const int kk = kb + int(threadIdx.x);
-    const uint32_t ns = kk < kv ? uint32_t((counts[kk] + per - 1) / per) : 0u;
-    uint32_t all;
-    const uint32_t lo = before + block_exclusive_scan<256>(ns, s_scan, &all);
-    if (uint32_t(slot) >= lo && uint32_t(slot) < lo + ns) {
-      s_found[0] = kk;
-      s_found[1] = slot - int(lo);
-    }
-    before += all;
-    if (uint32_t(slot) < before) break;
-  }
-  __syncthreads();
-  const int k = s_found[0];
-  if (k < 0) return;  // fewer shares than slots
-  const int split = s_found[1];
-  const int c0 = (blk / nblocks) * BW, n0 = (blk % nblocks) * BW;
   const int tid = threadIdx.x;
   const int wave = tid >> 6, lane = tid & 63;
+  const int64_t per = wg_per(wg_total(counts, kv, lane), target, STAGE);
+  int k = -1, split = 0;  // the offset whose shares hold `slot`, and which of them
+  // the launch's first wave leaves every offset's first share for the reduction
+  const bool writer = blockIdx.x == 0 && tid < 64;
+  int before = 0;
+  for (int kb = 0; kb < kv && (before <= slot || writer); kb += 64) {
+    const int ns = kb + lane < kv ? wg_count(counts[kb + lane], per) : 0;
+    int upto = ns;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int v = __shfl_up(upto, off, 64);
+      upto += lane >= off ? v : 0;
+    }
+    const int start = before + upto - ns;
+    const uint64_t mine = __ballot(slot >= start && slot < start + ns);
+    if (mine) {
+      const int l = __builtin_ctzll(mine);
+      k = kb + l;
+      split = slot - __shfl(start, l, 64);
+    }
+    if (writer && kb + lane < kv) first[kb + lane] = start;
+    before += __shfl(upto, 63, 64);
+  }
+  if (writer && lane == 0) first[kv] = before;
+  k = __builtin_amdgcn_readfirstlane(k);
+  split = __builtin_amdgcn_readfirstlane(split);
+  if (k < 0) return;  // fewer shares than slots
+  const int c0 = (blk / nblocks) * BW, n0 = (blk % nblocks) * BW;
   const int h = lane >> 5, l32 = lane & 31;
   const int ctile = (wave >> 1) * (BW / 2), ntile = (wave & 1) * (BW / 2);
   // staging role: pairs 2 pp and 2 pp + 1 of a stage and NV vectors of V
@@ -455,26 +470,21 @@ __global__ __launch_bounds__(256) void wgrad_partial(
 // part of the offset's shares, eight in flight, and the sums meet in LDS in
 // ascending share.  SPLIT: the partials hold the products of X's and G's
 // [hi | lo] halves ([2K][2C]), whose four values of an entry are added, in a
-// fixed order, into the fp32 dW.
+// fixed order, into the fp32 dW.  W = 4 stores its values together.  (A workgroup
+// of a 256 x 256 gradient has little to do: summing the counts in each took 14 us
+// where first[], an offset's first share, takes 6.)
 template <typename T, int W, bool SPLIT, int NW>
 __global__ __launch_bounds__(64 * NW) void wgrad_reduce(
-    const float* __restrict__ part, const int32_t* __restrict__ counts, int kv, int target,
-    int stage, int K, int C, T* __restrict__ dw) {
+    const float* __restrict__ part, const int32_t* __restrict__ first, int kv, int K, int C,
+    T* __restrict__ dw) {
   __shared__ float s_part[NW][64 * W];
-  __shared__ int64_t s_red[NW];
   const int k = int(blockIdx.y);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  int64_t total = 0;
-  for (int kk = threadIdx.x; kk < kv; kk += 64 * NW) total += counts[kk];
-  const int64_t per = wg_per(wg_block_sum<64 * NW>(total, s_red), target, stage);
-  int64_t lo = 0;  // the offset's first share
-  for (int kk = threadIdx.x; kk < k; kk += 64 * NW)
-    lo += (counts[kk] + per - 1) / per;
-  lo = wg_block_sum<64 * NW>(lo, s_red);
-  const int ns = int((counts[k] + per - 1) / per);
+  const int64_t lo = first[k];
+  const int ns = first[k + 1] - int(lo);
 
-  const int E = K * C;
-  const int e0 = (int(blockIdx.x) * 64 + lane) * W;
+  const uint32_t E = uint32_t(K) * uint32_t(C);  // (K, C < 65536)
+  const uint32_t e0 = (blockIdx.x * 64u + uint32_t(lane)) * W;
   const bool ok = e0 < E;
   const int each = (ns + NW - 1) / NW;
   const int w_lo = wave * each < ns ? wave * each : ns;
@@ -484,7 +494,7 @@ __global__ __launch_bounds__(64 * NW) void wgrad_reduce(
   constexpr int kParts = SPLIT ? 4 : 1;
   int64_t at[kParts];
   if constexpr (SPLIT) {
-    const int n = e0 / C, c = e0 % C;  // (W divides C)
+    const int64_t n = e0 / uint32_t(C), c = e0 % uint32_t(C);  // (W divides C)
 #pragma unroll
     for (int a = 0; a < 2; ++a)
 #pragma unroll
@@ -519,11 +529,12 @@ __global__ __launch_bounds__(64 * NW) void wgrad_reduce(
   __syncthreads();
   if (wave != 0 || !ok) return;
   for (int w = 1; w < NW; ++w) sum += *reinterpret_cast<const vec*>(&s_part[w][lane * W]);
+  using out_vec = __attribute__((ext_vector_type(W))) T;
+  out_vec o;
 #pragma unroll
-  for (int i = 0; i < W; ++i) {
-    const int e = e0 + i, n = e / C, c = e % C;
-    dw[(int64_t(n) * kv + k) * C + c] = from_f32<T>(sum[i]);
-  }
+  for (int i = 0; i < W; ++i) o[i] = from_f32<T>(sum[i]);
+  const int64_t n = e0 / uint32_t(C), c = e0 % uint32_t(C);
+  *reinterpret_cast<out_vec*>(dw + (n * kv + k) * C + c) = o;
 }
 
 // out [rows][parts * cols] bf16 from x [rows][cols] fp32: pattern 0 = [hi |
@@ -955,27 +966,52 @@ static int wgrad_block(int64_t C, int64_t K) { return C >= 128 && K >= 128 ? 128
 
 // Shares a call aims at, and the slots its partials need: an offset's last
 // share may be a short one, so there are at most kv more shares than aimed at.
-// The fewest that fill the chip: every share writes and reads a fp32 partial of
-// its block.  Split-bf16 operands, whose fp32 results are summed in one chain a
-// share, take at least 64 workgroups per offset, so that none is long.  Measured (us a call, 256 / 512 / 768 / 1024 / 1536 /
-// 2048 workgroups): urban 240k rows, 410k pairs, 64 -> 64 33.2 / 30.5 / 33.8 /
-// 35.4 / 37.1 / 42.4; k2 s2 64 -> 128 33.2 / 27.8 / 28.6 / 29.9 / 32.2 / 36.6;
-// 75k rows, 349k pairs, 256 -> 128 (128-wide blocks) 108 / 107 / 100 / 99 /
-// 108 / 117, 256 -> 256 189 / 183 / 165 / 166 / 166 / 176.
-static int wgrad_target(int64_t kv, int64_t C, int64_t K, int64_t n_rows, bool split) {
+// Every share writes and reads a fp32 partial of its block, so there are no
+// more than fill the chip, 512 workgroups for 64-wide blocks (two a CU) and
+// 1024 for 128-wide ones, and none beyond: with 512 aimed at, the offsets' short
+// shares came to up to 539, and the few past 512 ran by themselves (us, aimed at
+// 512 and 512 - kv, fp32 64 -> 64: dense 48^3 grid 504 and 376, 200k surface
+// rows 392 and 299; fp16 111 and 82, 102 and 81).  Where kv takes up most of
+// that, as many more rounds as leave half a round to share out.  A share has at
+// least 128 pairs if every entry of the table were one, 512 of 16 bits (dense
+// 10^3 grid fp16 256 -> 256 41 and 34).  Split-bf16 operands, whose fp32 results
+// are summed in one chain a share, take at least 64 workgroups per offset, so
+// that none is long.  Measured (us a call, 256 / 512 / 1024 / 2048 workgroups
+// aimed at): urban 240k rows, 410k pairs, 64 -> 64 fp16 31.3 / 28.4 / 32.6 / 39.8;
+// k2s2 64 -> 64 23.0 / 21.1 / 23.9 / 30.9; 75k surface rows, 349k pairs, 256 ->
+// 256 (128-wide blocks) 132 / 129 / 112 / 126.
+static int wgrad_target(int64_t kv, int64_t C, int64_t K, int64_t n_rows, int elem, bool split) {
   const int bw = wgrad_block(C, K);
-  int64_t wgs = bw == 128 ? 1024 : 512;
-  if (split && wgs < 64 * kv) wgs = 64 * kv;
-  int64_t t = cdiv(wgs, cdiv(C, bw) * cdiv(K, bw));
-  const int64_t by_len = cdiv(n_rows * kv, 128);  // a stage of pairs each, if every entry were one
+  const int64_t blocks = cdiv(C, bw) * cdiv(K, bw);
+  const int64_t wgs = bw == 128 ? 1024 : 512;
+  int64_t t;
+  if (split) {
+    t = cdiv(wgs < 64 * kv ? 64 * kv : wgs, blocks);
+  } else {
+    const int64_t round = wgs / blocks < 1 ? 1 : wgs / blocks;
+    t = cdiv(kv + round / 2, round) * round - kv;
+  }
+  const int64_t by_len = cdiv(n_rows * kv, elem == SP_F32 || split ? 128 : 512);
   if (t > by_len) t = by_len;
   return int(t < 1 ? 1 : t);
 }
 // Blocks up to this many values an offset are reduced by 16 waves a workgroup
 // (few workgroups, and a dense offset has most of the shares), larger ones by 4.
 constexpr int64_t kWgWideReduce = 8192;
-static int64_t wgrad_slots(int64_t kv, int64_t C, int64_t K, int64_t n_rows, bool split) {
-  return wgrad_target(kv, C, K, n_rows, split) + kv;
+// Workspace: the offsets' first shares [kv + 1], then the partials.
+struct WgLayout {
+  int target;
+  int64_t slots;
+  size_t part_off, total;
+};
+static WgLayout wgrad_layout(int64_t kv, int64_t C, int64_t K, int64_t n_rows, int elem,
+                             bool split) {
+  WgLayout l;
+  l.target = wgrad_target(kv, C, K, n_rows, elem, split);
+  l.slots = l.target + kv;
+  l.part_off = align_up(size_t(kv + 1) * sizeof(int32_t), 256);
+  l.total = l.part_off + align_up(size_t(l.slots) * size_t(K * C) * sizeof(float), 256);
+  return l;
 }
 
 // ---- the forward without a caller workspace (sp_conv_fwd_noalloc) ---------
@@ -1106,8 +1142,10 @@ int sp_conv_dgrad(const void* g, int32_t dtype, int64_t n_out, int64_t K, const 
 }
 
 size_t sp_wgrad_workspace_size(int64_t K, int64_t kv, int64_t C, int64_t n_rows) {
-  // (the larger of the two shares' counts: the type is not known here)
-  return align_up(size_t(wgrad_slots(kv, C, K, n_rows, true)) * size_t(K * C) * sizeof(float), 256);
+  // (the most of any type: it is not known here)
+  const size_t a = wgrad_layout(kv, C, K, n_rows, SP_F32, false).total;
+  const size_t b = wgrad_layout(kv, C, K, n_rows, SP_BF16, true).total;
+  return a > b ? a : b;
 }
 
 int sp_conv_wgrad(const void* x, int64_t n_in, const void* g, int64_t n_out, int32_t dtype,
@@ -1126,12 +1164,13 @@ int sp_conv_wgrad(const void* x, int64_t n_in, const void* g, int64_t n_out, int
   SP_CHECK_ARG(Kg * Cg < (int64_t(1) << 30) && row_stride < (int64_t(1) << 31),
                "wgrad: weight or table too large");
   const int elem = split ? SP_BF16 : dtype;
-  const int64_t slots = wgrad_slots(kv, Cg, Kg, row_stride, split);
-  const int target = wgrad_target(kv, Cg, Kg, row_stride, split);
+  const WgLayout l = wgrad_layout(kv, Cg, Kg, row_stride, elem, split);
+  const int64_t slots = l.slots;
   const size_t need = sp_wgrad_workspace_size(Kg, kv, Cg, row_stride);
   if (!ws || ws_bytes < need)
     return set_error(SP_ERR_WORKSPACE, "wgrad: workspace %zu < %zu", ws_bytes, need);
-  float* part = static_cast<float*>(ws);
+  int32_t* first = static_cast<int32_t*>(ws);
+  float* part = reinterpret_cast<float*>(static_cast<char*>(ws) + l.part_off);
   const int64_t es = elem == SP_F32 ? 4 : 2;
   const int64_t xb = n_in * Cg * es, gb = n_out * Kg * es;
   if (xb >= int64_t(kOob) || gb >= int64_t(kOob))
@@ -1145,7 +1184,9 @@ int sp_conv_wgrad(const void* x, int64_t n_in, const void* g, int64_t n_out, int
   const int64_t nwg = 8 * cdiv(slots, 8) * cblocks * nblocks;
   SP_CHECK_ARG(nwg <= kMaxGridX, "wgrad: grid too large");
   const dim3 grid{unsigned(nwg), 1u, 1u};
-  const int rw = C % 4 == 0 ? 4 : 1;
+  // four values a lane where their store is aligned
+  const size_t out_es = split || elem == SP_F32 ? 4 : 2;
+  const int rw = C % 4 == 0 && reinterpret_cast<uintptr_t>(dw) % (4 * out_es) == 0 ? 4 : 1;
   const dim3 rgrid{unsigned(cdiv(K * C, 64 * rw)), unsigned(kv)};
   auto run = [&](auto tag) {
     using T = decltype(tag);
@@ -1157,16 +1198,14 @@ int sp_conv_wgrad(const void* x, int64_t n_in, const void* g, int64_t n_out, int
     const Kern kern = bw == 128 ? k128[vec] : k64[vec];
     kern<<<grid, 256, 0, s>>>(static_cast<const T*>(x), n_in, static_cast<const T*>(g), n_out,
                               int(Cg), int(Kg), int(kv), in_rows, out_rows, counts, row_stride,
-                              target, int(slots), part, uint32_t(xb), uint32_t(gb), cblocks,
-                              nblocks);
-    const int stage = bw == 128 ? WgShape<T, 128>::kStage : WgShape<T, 64>::kStage;
+                              l.target, int(slots), part, first, uint32_t(xb), uint32_t(gb),
+                              cblocks, nblocks);
     auto reduce = [&](auto out, auto is_split, auto waves) {
       using O = decltype(out);
       constexpr bool SPL = decltype(is_split)::value;
       constexpr int NW = decltype(waves)::value;
       auto red = rw == 4 ? wgrad_reduce<O, 4, SPL, NW> : wgrad_reduce<O, 1, SPL, NW>;
-      red<<<rgrid, 64 * NW, 0, s>>>(part, counts, int(kv), target, stage, int(K), int(C),
-                                    static_cast<O*>(dw));
+      red<<<rgrid, 64 * NW, 0, s>>>(part, first, int(kv), int(K), int(C), static_cast<O*>(dw));
     };
     auto with_waves = [&](auto out, auto is_split) {
       if (K * C <= kWgWideReduce)
