@@ -365,6 +365,7 @@ int sp_split_bf16x3(const float* x, int64_t rows, int64_t cols, int32_t pattern,
  * dW[n, k, c] = sum_{p < counts[k]} X[in_rows[k, p], c] * G[out_rows[k, p], n].
  * X [n_in, C], G [n_out, K]; in_rows/out_rows [kv, row_stride].  fp32 partials of
  * shares of the pairs, summed in a fixed order (deterministic).  dW [K, kv, C] in dtype.
+ * ws may start at any byte, dw at any element.
  * dtype SP_BF16X3: x [n_in, 2C]
  * and g [n_out, 2K] are the bf16 [hi | lo] halves of fp32 tensors (sp_split_bf16x3
  * pattern 2), dW is fp32 (the four half products summed), and the workspace is

@@ -998,7 +998,8 @@ static int wgrad_target(int64_t kv, int64_t C, int64_t K, int64_t n_rows, int el
 // Blocks up to this many values an offset are reduced by 16 waves a workgroup
 // (few workgroups, and a dense offset has most of the shares), larger ones by 4.
 constexpr int64_t kWgWideReduce = 8192;
-// Workspace: the offsets' first shares [kv + 1], then the partials.
+// Workspace, from its first 16-byte boundary (the partials move in 16-byte pieces): the
+// offsets' first shares [kv + 1], then the partials.
 struct WgLayout {
   int target;
   int64_t slots;
@@ -1010,7 +1011,7 @@ static WgLayout wgrad_layout(int64_t kv, int64_t C, int64_t K, int64_t n_rows, i
   l.target = wgrad_target(kv, C, K, n_rows, elem, split);
   l.slots = l.target + kv;
   l.part_off = align_up(size_t(kv + 1) * sizeof(int32_t), 256);
-  l.total = l.part_off + align_up(size_t(l.slots) * size_t(K * C) * sizeof(float), 256);
+  l.total = 16 + l.part_off + align_up(size_t(l.slots) * size_t(K * C) * sizeof(float), 256);
   return l;
 }
 
@@ -1169,8 +1170,9 @@ int sp_conv_wgrad(const void* x, int64_t n_in, const void* g, int64_t n_out, int
   const size_t need = sp_wgrad_workspace_size(Kg, kv, Cg, row_stride);
   if (!ws || ws_bytes < need)
     return set_error(SP_ERR_WORKSPACE, "wgrad: workspace %zu < %zu", ws_bytes, need);
-  int32_t* first = static_cast<int32_t*>(ws);
-  float* part = reinterpret_cast<float*>(static_cast<char*>(ws) + l.part_off);
+  char* base = reinterpret_cast<char*>((reinterpret_cast<uintptr_t>(ws) + 15) & ~uintptr_t(15));
+  int32_t* first = reinterpret_cast<int32_t*>(base);
+  float* part = reinterpret_cast<float*>(base + l.part_off);
   const int64_t es = elem == SP_F32 ? 4 : 2;
   const int64_t xb = n_in * Cg * es, gb = n_out * Kg * es;
   if (xb >= int64_t(kOob) || gb >= int64_t(kOob))

@@ -122,3 +122,39 @@ def test_shares_match_fp64(kv, n, C, K, density, dtype):
         ref, mag = gi.T @ xi, gi.abs().T @ xi.abs()
         bound = unit * ref.abs() + (o.numel() + 1) * 2.0 ** -24 * mag * (1 + unit) + 1e-30
         assert ((dw[:, k].double() - ref).abs() <= bound).all(), f"offset {k}"
+
+
+def _call(x, go, tab, K, ws, dw):
+    """sp_conv_wgrad with the caller's own buffers."""
+    from spconv_triton.pytorch._impl import _lib
+    from spconv_triton.pytorch._impl.gemm import compacted_signal
+
+    in_rows, out_rows, counts = compacted_signal(tab)
+    kv, n = tab.shape
+    _lib.check(_lib.lib().sp_conv_wgrad(
+        _lib.ptr(x), x.shape[0], _lib.ptr(go), n, _lib.dtype_code(x.dtype), x.shape[1], K, kv,
+        _lib.ptr(in_rows), _lib.ptr(out_rows), _lib.ptr(counts), n, _lib.ptr(dw), _lib.ptr(ws),
+        ws.numel(), _lib.stream_of(x.device)), "sp_conv_wgrad")
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.float32])
+@pytest.mark.parametrize("ws_off,dw_off", [(0, 0), (4, 0), (0, 1), (12, 3), (1, 2)])
+def test_buffers_at_any_address(dtype, ws_off, dw_off):
+    """The workspace may start at any byte and dW at any element; nothing is written past them."""
+    from spconv_triton.pytorch._impl import _lib
+    from spconv_triton.pytorch._impl.gemm import conv_backward_weight
+
+    kv, n, C, K = 5, 700, 20, 24
+    tab = torch.from_numpy(_table(kv, n, n, [0.5, 0.1], 3)).to(DEV)
+    g = torch.Generator(device=DEV)
+    g.manual_seed(1)
+    x = torch.randn(n, C, generator=g, device=DEV).to(dtype)
+    go = torch.randn(n, K, generator=g, device=DEV).to(dtype)
+    size = _lib.lib().sp_wgrad_workspace_size(K, kv, C, n)
+    ws = torch.full((size + 64,), 0xA5, dtype=torch.uint8, device=DEV)
+    out = torch.full((K * kv * C + 8,), 7.0, dtype=dtype, device=DEV)
+    _call(x, go, tab, K, ws[ws_off:ws_off + size], out[dw_off:])
+    want = conv_backward_weight(x, go, tab, (K, kv, C)).view(-1)
+    assert torch.equal(out[dw_off:dw_off + want.numel()], want)
+    assert (out[:dw_off] == 7).all() and (out[dw_off + want.numel():] == 7).all()
+    assert (ws[:ws_off] == 0xA5).all() and (ws[ws_off + size:] == 0xA5).all()
