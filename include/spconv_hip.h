@@ -368,9 +368,11 @@ int sp_split_bf16x3(const float* x, int64_t rows, int64_t cols, int32_t pattern,
  * ws may start at any byte, dw at any element.
  * dtype SP_BF16X3: x [n_in, 2C]
  * and g [n_out, 2K] are the bf16 [hi | lo] halves of fp32 tensors (sp_split_bf16x3
- * pattern 2), dW is fp32 (the four half products summed), and the workspace is
- * sp_wgrad_workspace_size(2K, kv, 2C, n_rows).
+ * pattern 2) and dW is fp32 (the four half products summed).
+ * Workspace: sp_conv_wgrad_workspace (0: no such dtype); sp_wgrad_workspace_size is the most
+ * of any type, with 2K and 2C for SP_BF16X3.  n_rows is the row_stride.
  * Replaces conv_backward_weight + _dweight_masked_kernel, gemm.py:324-453, :634-713. */
+size_t sp_conv_wgrad_workspace(int32_t dtype, int64_t C, int64_t K, int64_t kv, int64_t n_rows);
 size_t sp_wgrad_workspace_size(int64_t K, int64_t kv, int64_t C, int64_t n_rows);
 int sp_conv_wgrad(const void* x, int64_t n_in, const void* g, int64_t n_out, int32_t dtype,
                   int64_t C, int64_t K, int64_t kv, const int32_t* in_rows,

@@ -1149,6 +1149,14 @@ size_t sp_wgrad_workspace_size(int64_t K, int64_t kv, int64_t C, int64_t n_rows)
   return a > b ? a : b;
 }
 
+size_t sp_conv_wgrad_workspace(int32_t dtype, int64_t C, int64_t K, int64_t kv, int64_t n_rows) {
+  if (!gemm_dtype_ok(dtype) && dtype != SP_BF16X3) return 0;
+  const bool split = dtype == SP_BF16X3;
+  return wgrad_layout(kv, split ? 2 * C : C, split ? 2 * K : K, n_rows, split ? SP_BF16 : dtype,
+                      split)
+      .total;
+}
+
 int sp_conv_wgrad(const void* x, int64_t n_in, const void* g, int64_t n_out, int32_t dtype,
                   int64_t C, int64_t K, int64_t kv, const int32_t* in_rows,
                   const int32_t* out_rows, const int32_t* counts, int64_t row_stride, void* dw,
@@ -1167,9 +1175,8 @@ int sp_conv_wgrad(const void* x, int64_t n_in, const void* g, int64_t n_out, int
   const int elem = split ? SP_BF16 : dtype;
   const WgLayout l = wgrad_layout(kv, Cg, Kg, row_stride, elem, split);
   const int64_t slots = l.slots;
-  const size_t need = sp_wgrad_workspace_size(Kg, kv, Cg, row_stride);
-  if (!ws || ws_bytes < need)
-    return set_error(SP_ERR_WORKSPACE, "wgrad: workspace %zu < %zu", ws_bytes, need);
+  if (!ws || ws_bytes < l.total)
+    return set_error(SP_ERR_WORKSPACE, "wgrad: workspace %zu < %zu", ws_bytes, l.total);
   char* base = reinterpret_cast<char*>((reinterpret_cast<uintptr_t>(ws) + 15) & ~uintptr_t(15));
   int32_t* first = reinterpret_cast<int32_t*>(base);
   float* part = reinterpret_cast<float*>(base + l.part_off);

@@ -129,6 +129,7 @@ _SIGNATURES = {
     "sp_conv_dgrad": (ctypes.c_int, [_P, _I32, _I64, _I64, _P, _I32, _I64, _I64, _P, _I64, _P,
                                      _P, _P, _P, _SZ, _P]),
     "sp_split_bf16x3": (ctypes.c_int, [_P, _I64, _I64, _I32, _P, _P]),
+    "sp_conv_wgrad_workspace": (_SZ, [_I32, _I64, _I64, _I64, _I64]),
     "sp_wgrad_workspace_size": (_SZ, [_I64, _I64, _I64, _I64]),
     "sp_conv_wgrad": (ctypes.c_int, [_P, _I64, _P, _I64, _I32, _I64, _I64, _I64, _P, _P, _P,
                                      _I64, _P, _P, _SZ, _P]),

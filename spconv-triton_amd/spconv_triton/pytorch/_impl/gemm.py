@@ -665,9 +665,7 @@ def conv_backward_weight(features: torch.Tensor, grad_out: torch.Tensor, pair_fw
     dt = _lib.dtype_code(x.dtype)
     if _tf32(x):  # split-bf16 halves [hi | lo]; the fp32 dW sums their four products
         x, g, dt = split_bf16(x, 2), split_bf16(g, 2), _lib.SP_BF16X3
-        ws = _lib.workspace(L.sp_wgrad_workspace_size(2 * K, kv, 2 * C, stride), x.device)
-    else:
-        ws = _lib.workspace(L.sp_wgrad_workspace_size(K, kv, C, stride), x.device)
+    ws = _lib.workspace(L.sp_conv_wgrad_workspace(dt, C, K, kv, stride), x.device)
     _lib.check(L.sp_conv_wgrad(_lib.ptr(x), x.shape[0], _lib.ptr(g), n_out,
                                dt, C, K, kv, _lib.ptr(in_rows),
                                _lib.ptr(out_rows), _lib.ptr(counts), stride, _lib.ptr(dw),

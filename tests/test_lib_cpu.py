@@ -104,6 +104,28 @@ def test_workspace_queries_and_bad_geometry():
     assert b"thin_tiles" in L.sp_last_error()
 
 
+def test_wgrad_workspace_follows_the_type():
+    """Partials for the shares a call of that type can have: a share holds at least 512 pairs of a
+    16-bit table if every entry is one (a fp32 table's 128), and there is one short share an
+    offset."""
+    from spconv_triton.pytorch._impl import _lib
+
+    L = _lib.load_library()
+    mb = 1 << 20
+    f16, bf16, f32, x3 = _lib.SP_F16, _lib.SP_BF16, _lib.SP_F32, _lib.SP_BF16X3
+    for kv, C, K, n in ((27, 64, 64, 200000), (27, 256, 256, 1000), (343, 64, 64, 50000),
+                        (8, 16, 24, 1), (27, 130, 200, 3000)):
+        by_type = {dt: L.sp_conv_wgrad_workspace(dt, C, K, kv, n) for dt in (f16, bf16, f32)}
+        assert by_type[f16] == by_type[bf16] <= by_type[f32]
+        assert max(by_type.values()) <= L.sp_wgrad_workspace_size(K, kv, C, n)
+        assert 0 < (L.sp_conv_wgrad_workspace(x3, C, K, kv, n)
+                    <= L.sp_wgrad_workspace_size(2 * K, kv, 2 * C, n))
+    assert L.sp_conv_wgrad_workspace(f16, 64, 64, 27, 200000) < 9 * mb
+    assert L.sp_conv_wgrad_workspace(f16, 256, 256, 27, 1000) < 21 * mb
+    assert L.sp_conv_wgrad_workspace(f16, 64, 64, 343, 50000) < 23 * mb
+    assert L.sp_conv_wgrad_workspace(_lib.SP_F64, 64, 64, 27, 1000) == 0
+
+
 def test_error_mapping():
     from spconv_triton.pytorch._impl import _lib
 
