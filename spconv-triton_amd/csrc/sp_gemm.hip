@@ -1170,8 +1170,6 @@ int sp_conv_wgrad(const void* x, int64_t n_in, const void* g, int64_t n_out, int
   const bool split = dtype == SP_BF16X3;
   const int64_t Cg = split ? 2 * C : C, Kg = split ? 2 * K : K;
   SP_CHECK_ARG(Kg < 65536 && Cg < 65536 && kv < 65536, "wgrad: channel/kernel size too large");
-  SP_CHECK_ARG(Kg * Cg < (int64_t(1) << 30) && row_stride < (int64_t(1) << 31),
-               "wgrad: weight or table too large");
   const int elem = split ? SP_BF16 : dtype;
   const WgLayout l = wgrad_layout(kv, Cg, Kg, row_stride, elem, split);
   const int64_t slots = l.slots;

@@ -158,3 +158,20 @@ def test_buffers_at_any_address(dtype, ws_off, dw_off):
     assert torch.equal(out[dw_off:dw_off + want.numel()], want)
     assert (out[:dw_off] == 7).all() and (out[dw_off + want.numel():] == 7).all()
     assert (ws[:ws_off] == 0xA5).all() and (ws[ws_off + size:] == 0xA5).all()
+
+
+def test_weights_of_a_billion_values():
+    """K * C = 2^30: entries are counted in 32 unsigned bits, their addresses in 64."""
+    from spconv_triton.pytorch._impl.gemm import conv_backward_weight
+
+    C = K = 32768
+    g = torch.Generator(device=DEV)
+    g.manual_seed(2)
+    x = torch.randint(-2, 3, (5, C), generator=g, device=DEV).half()
+    go = torch.randint(-1, 2, (5, K), generator=g, device=DEV).half()
+    tab = torch.tensor([[3, -1, 0, 4, 2]], dtype=torch.int32, device=DEV)
+    dw = conv_backward_weight(x, go, tab, (K, 1, C)).view(K, C)
+    o = torch.tensor([0, 2, 3, 4], device=DEV)
+    for n0 in range(0, K, 4096):
+        ref = go[o, n0:n0 + 4096].float().T.contiguous() @ x[tab[0, o].long()].float()
+        assert torch.equal(dw[n0:n0 + 4096], ref.half())
