@@ -124,6 +124,27 @@ def test_point_to_voxel_list_sizes(n, most, max_pts):
     _eq(res, _orc(ctor, pts), f"n {n} most {most}")
 
 
+@pytest.mark.parametrize("n,run", [(1, 1), (63, 63), (257, 64), (5000, 5000), (5000, 3), (3000, 40),
+                                   (40_000, 32)])
+@pytest.mark.parametrize("shuffled", [False, True])
+def test_point_to_voxel_points_of_a_wave_share_voxels(n, run, shuffled):
+    """Runs of points in one voxel (all of them at the longest), some out of range between."""
+    rng = np.random.default_rng(n + run)
+    cell = np.arange(n) // run
+    if shuffled:
+        cell = rng.permutation(cell)
+    pts = rng.random((n, 4)).astype(np.float32)
+    pts[:, 0] = (cell % 50) + rng.random(n) * 0.9
+    pts[:, 1] = (cell // 50 % 50) + rng.random(n) * 0.9
+    pts[:, 2] = 0.5
+    if n > 1:
+        pts[rng.random(n) < 0.05, 1] = -3.0
+    pts = torch.from_numpy(pts)
+    ctor = dict(vsize_xyz=[1, 1, 1], coors_range_xyz=[0, 0, 0, 50, 50, 4], num_point_features=4,
+                max_num_voxels=900, max_num_points_per_voxel=20)
+    _eq(_p2v(ctor, pts)[1], _orc(ctor, pts), f"{n} points, runs of {run}")
+
+
 def test_point_to_voxel_empty_mean():
     """empty_mean fills empty slots with the voxel's mean (the sum over all
     slots, in slot order, over the clamped count: one rounding order of the
