@@ -624,10 +624,13 @@ def conv_backward_input(grad_out: torch.Tensor, filters_krsc: torch.Tensor,
 def compacted_signal(pair_fwd: torch.Tensor):
     """Per-offset (input row, output row) lists of a gather table, output rows
     ascending -- the reference's ``valid_signal`` (gemm.py:661-669) in a
-    per-offset slotted layout.  Memoised on the table tensor."""
+    per-offset slotted layout.  Memoised on the table tensor; rebuilt if the
+    table is modified in place."""
     cached = getattr(pair_fwd, "_spconv_triton_dw_sig", None)
-    if cached is not None:
-        return cached
+    # (inference tensors have no version)
+    stamp = (None if pair_fwd.is_inference() else pair_fwd._version, pair_fwd.data_ptr())
+    if cached is not None and cached[0] == stamp:
+        return cached[1]
     pf = pair_fwd.contiguous()
     kv, n = pf.shape
     device = pf.device
@@ -640,7 +643,7 @@ def compacted_signal(pair_fwd: torch.Tensor):
                                   _lib.ptr(counts), _lib.ptr(ws), ws.numel(),
                                   _lib.stream_of(device)), "sp_compact_pairs")
     sig = (in_rows, out_rows, counts)
-    pair_fwd._spconv_triton_dw_sig = sig
+    pair_fwd._spconv_triton_dw_sig = (stamp, sig)
     return sig
 
 

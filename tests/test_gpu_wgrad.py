@@ -160,6 +160,20 @@ def test_buffers_at_any_address(dtype, ws_off, dw_off):
     assert (ws[:ws_off] == 0xA5).all() and (ws[ws_off + size:] == 0xA5).all()
 
 
+def test_a_table_edited_in_place_is_compacted_again():
+    from spconv_triton.pytorch._impl.gemm import compacted_signal, conv_backward_weight
+
+    kv, n, C, K = 9, 500, 16, 16
+    tab = torch.from_numpy(_table(kv, n, n, [0.4], 5)).to(DEV)
+    x = torch.randn(n, C, device=DEV)
+    go = torch.randn(n, K, device=DEV)
+    conv_backward_weight(x, go, tab, (K, kv, C))
+    assert compacted_signal(tab)[2] is compacted_signal(tab)[2]
+    tab[:, ::3] = -1
+    want = conv_backward_weight(x, go, tab.clone(), (K, kv, C))
+    assert torch.equal(conv_backward_weight(x, go, tab, (K, kv, C)), want)
+
+
 def test_weights_of_a_billion_values():
     """K * C = 2^30: entries are counted in 32 unsigned bits, their addresses in 64."""
     from spconv_triton.pytorch._impl.gemm import conv_backward_weight
