@@ -5,7 +5,6 @@
 #pragma once
 
 #include <mutex>
-#include <vector>
 
 #include "sp_common.h"
 
@@ -14,9 +13,12 @@ namespace sp {
 // Small pinned host buffers that kernels write their counts to, kept between
 // calls (one per call in flight, whatever the thread or device): a copy of the
 // counts from device memory costs a launch and ~4 us before the host goes on.
+// At most kIdle of 256 bytes are kept; what more calls in flight needed is freed.
 struct PinnedPool {
+  static constexpr int kIdle = 64;
   std::mutex m;
-  std::vector<void*> idle;
+  void* idle[kIdle];
+  int n = 0;
 };
 inline PinnedPool& pinned_pool() {
   static PinnedPool* p = new PinnedPool;  // (outlives the threads that return buffers to it)
@@ -28,9 +30,8 @@ class PinnedCounts {
   int take() {
     {
       std::lock_guard<std::mutex> lock(pinned_pool().m);
-      if (!pinned_pool().idle.empty()) {
-        p_ = pinned_pool().idle.back();
-        pinned_pool().idle.pop_back();
+      if (pinned_pool().n > 0) {
+        p_ = pinned_pool().idle[--pinned_pool().n];
         return SP_OK;
       }
     }
@@ -39,8 +40,14 @@ class PinnedCounts {
   }
   ~PinnedCounts() {
     if (!p_) return;
-    std::lock_guard<std::mutex> lock(pinned_pool().m);
-    pinned_pool().idle.push_back(p_);
+    {
+      std::lock_guard<std::mutex> lock(pinned_pool().m);
+      if (pinned_pool().n < PinnedPool::kIdle) {
+        pinned_pool().idle[pinned_pool().n++] = p_;
+        return;
+      }
+    }
+    (void)hipHostFree(p_);
   }
   uint64_t* data() const { return static_cast<uint64_t*>(p_); }
 

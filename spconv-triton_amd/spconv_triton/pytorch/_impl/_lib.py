@@ -2,8 +2,9 @@
 
 The symbols and argument meanings are those declared in ``include/spconv_hip.h``.
 Every call passes raw device pointers of torch tensors and torch's current
-HIP stream; the library never allocates, so workspaces come from torch's
-caching allocator.
+HIP stream; the library allocates no device memory, so workspaces come from
+torch's caching allocator.  (It keeps up to 64 pinned host buffers of 256
+bytes, one per call in flight, for counts that kernels write to the host.)
 
 There is no fallback: if the library is missing, or a tensor is not on the
 GPU, the call raises.  The library must bind to the same HIP runtime as

@@ -50,3 +50,46 @@ def test_bitmap_rulebook_matches_oracle(ci):
         bwd = np.where(exp[3] < m, exp[3], -1)
         np.testing.assert_array_equal(res[3].cpu().numpy(), bwd)
         assert int((res[2] >= 0).sum()) == int((bwd >= 0).sum())
+
+
+def test_rulebooks_of_many_threads_at_once():
+    """Each call in flight has its own counts, whatever the thread, stream or size."""
+    import threading
+
+    from spconv_triton.core import ConvAlgo
+    from spconv_triton.pytorch import ops
+
+    rng = np.random.default_rng(11)
+    shape = [16, 40, 48]
+
+    def build(it):
+        return ops.get_indice_pairs_implicit_gemm(
+            it, 1, shape, ConvAlgo.MaskImplicitGemm, [3] * 3, [2] * 3, [1] * 3, [1] * 3, [0] * 3,
+            False, False, is_train=True)
+
+    inputs, want = [], []
+    for n in (5, 90, 400, 1500, 3000, 4000, 6000, 9000):
+        lin = np.sort(rng.choice(int(np.prod(shape)), size=n, replace=False))
+        idx = np.concatenate([np.zeros((n, 1)), np.stack(np.unravel_index(lin, shape), 1)], 1)
+        inputs.append(torch.from_numpy(idx.astype(np.int32)).to(DEV))
+        res = build(inputs[-1])
+        want.append([res[0].cpu(), res[2].cpu(), res[3].cpu()])
+    torch.cuda.synchronize()
+    errors = []
+
+    def work(i):
+        try:
+            with torch.cuda.stream(torch.cuda.Stream()):
+                for _ in range(20):
+                    res = build(inputs[i])
+                    got = [res[0].cpu(), res[2].cpu(), res[3].cpu()]
+                    assert all(torch.equal(a, b) for a, b in zip(got, want[i]))
+        except BaseException as e:  # (an assertion in a thread would be lost)
+            errors.append((i, repr(e)))
+
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(len(inputs))]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors
