@@ -23,7 +23,6 @@
 //    is written back into its hash slot as its output row.
 #include <type_traits>
 
-
 #include "sp_common.h"
 #include "sp_hash.h"
 #include "sp_lookback.h"
@@ -1068,10 +1067,11 @@ static int run_brick_subm(const int32_t* indices, int64_t n, const GeomDev& d, T
 // With int32 keys and an output key volume of at most kBitmapCellsPerRow cells
 // per input row, one bit per output cell replaces the hash, the key sort and
 // the ranking.  Candidates set their cell's bit; an exclusive scan of the
-// 32-bit words' popcounts gives each word's first rank; a key's output row is
+// 64-cell words' popcounts gives each word's first rank; a key's output row is
 // that prefix plus the popcount of its word's lower bits, i.e. its rank in
 // ascending key order (torch.unique's order, as the hash path's sort gives).
-// The set bits, read in word order, are the sorted unique keys themselves.
+// The pairs' pass ranks its keys and writes the output rows' coordinates; the
+// bitmap is not read back.
 // The bitmap's passes cost in proportion to the output volume, the hash
 // path's in proportion to the candidates (n * kv, each an insert with probing,
 // then a radix sort and a ranking pass): the bitmap is taken up to 4096 cells
@@ -1098,7 +1098,7 @@ static bool conv_bitmap(const GeomDev& g, int64_t n, bool key64) {
 constexpr int kBitmapChunk = 8192;  // 32-bit words a workgroup of the scan covers
 struct BitmapWs {
   uint32_t* bits;     // [words] occupancy, bit key % 32 of word key / 32
-  uint32_t* prefix;   // [words / 2] set bits in the 64-cell words before (written for
+  uint32_t* prefix;   // [words64] set bits in the 64-cell words before (written for
                       // 4 words at a time, and not where all 4 are empty)
   uint32_t* meta;     // [64]
   uint64_t* state;    // [chunks]
@@ -1109,7 +1109,7 @@ template <class W>
 static void bitmap_layout(W& w, const GeomDev& g, BitmapWs* out) {
   const int64_t words = cdiv(g.batch * prod_shape(g.out_shape, g.ndim), 32);
   auto* bits = w.template take<uint32_t>(size_t(words));
-  auto* prefix = w.template take<uint32_t>(size_t(words));
+  auto* prefix = w.template take<uint32_t>(size_t(words));  // (callers know the size: half is used)
   auto* meta = w.template take<uint32_t>(64);
   void* state = w.template take<char>(scan_workspace_bytes(words));  // 4 bytes per 4096 words
   static_assert(kBitmapChunk * 4 >= 8 * kScanChunk, "a chunk's state fits");
