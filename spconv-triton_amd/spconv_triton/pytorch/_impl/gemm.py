@@ -520,7 +520,8 @@ def _gemm(a: torch.Tensor, filters: torch.Tensor, bias, transpose: bool, pairs: 
     use_plan = _use_plan(M, C, K)
     variant = row_order_variant(pairs, a.shape[0], K * C, use_plan,
                                 fp32=a.dtype == torch.float32 and not split)
-    if variant is None and _narrow(C if transpose else K, a.shape[1], a.dtype, out.dtype):
+    if (use_plan and variant is None
+            and _narrow(C if transpose else K, a.shape[1], a.dtype, out.dtype)):
         use_plan = False
     if split:  # the GEMM's reduction dimension is tripled
         K, C = (3 * K, C) if transpose else (K, 3 * C)
