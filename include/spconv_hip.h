@@ -381,8 +381,8 @@ int sp_conv_wgrad(const void* x, int64_t n_in, const void* g, int64_t n_out, int
 
 /* Eval-mode BatchNorm over rows [rows, C] (f16/bf16/f32):
  * out = fma(weight * (x - mean), rsqrt(var + eps), bias) in fp32, rounded, and max(out, 0) with
- * relu (a NaN stays): bit for bit what torch's modules give.  mean, var, weight and bias [C] in param_dtype (the rows' type or fp32);
- * weight and bias nullable (1 and 0).  The reference runs torch's modules here. */
+ * relu (a NaN stays): bit for bit what torch's modules give.  mean, var, weight and bias [C]
+ * in param_dtype (the rows' type or fp32); weight and bias nullable (1 and 0).  The reference runs torch's modules here. */
 int sp_batchnorm_eval(const void* x, int32_t dtype, int64_t rows, int64_t C, const void* mean,
                       const void* var, const void* weight, const void* bias, int32_t param_dtype,
                       float eps, int32_t relu, void* out, void* stream);
